@@ -172,6 +172,18 @@ typedef struct hrt_mm_reduce_args {
   uint32_t has_bias, pad;
 } hrt_mm_reduce_args;
 
+/* "mm_splitk_{bf16,f16}" — the product of "mm_mfma_{bf16,f16}" (flags 0) with K split over fp32 partial products
+ * where that is faster, and their ordered sum, in one call (no counterpart in the reference).  ws: at least
+ * hrt_mm_workspace(&mm) floats, 16-byte aligned, ws_floats of them; 0 floats: the plain product. */
+typedef struct hrt_mm_splitk_args {
+  hrt_mm_args mm;
+  uint64_t ws;
+  int64_t ws_floats;
+} hrt_mm_splitk_args;
+/* fp32 elements of workspace "mm_splitk_*" uses for this product (0: it is not split; -1: its operands
+ * are not aligned as the split kernel needs).  A pure host function of the sizes, strides and alignments. */
+int64_t hrt_mm_workspace(const hrt_mm_args* mm);
+
 /* "mm_dq8_{bf16,f16}" — fused int8 weight-only linear (no reference counterpart; composes
  * csrc/ops_quant.cpp:34-59 with csrc/ops_mm.cpp:61-175):
  *   y[m, n] = alpha * sum_k x[m, k] * deq(q)[n, k] + beta * bias[n]
@@ -180,7 +192,9 @@ typedef struct hrt_mm_reduce_args {
  * nblocks = ceil(K / 64); bias: [N] (if has_bias); y: [M, N] contiguous, dtype of x.
  * ws (optional, 0 = none): 16-byte aligned workspace of N * K elements of x's dtype.  For large M (the
  * weights would otherwise be converted once per 256-row block of x) the weights are dequantized into it
- * once and the product runs on them; the values are the same either way. */
+ * once and the product runs on them; the values are the same either way.  For small M it may hold fp32 partial
+ * products over slices of K, added in order (a reduction order of its own).  hrt_mm_dq8_workspace gives the
+ * elements that help a call: N * K or 0. */
 typedef struct hrt_mm_dq8_args {
   uint64_t x, q, scale, bias, y;
   int64_t M, N, K, nblocks;
@@ -189,6 +203,7 @@ typedef struct hrt_mm_dq8_args {
   uint32_t has_bias, flags;
   uint64_t ws;
 } hrt_mm_dq8_args;
+int64_t hrt_mm_dq8_workspace(const hrt_mm_dq8_args* args);
 
 /* Fused scaled-dot-product attention, non-causal, no mask, D <= 128 (vkrt/shaders/attn.comp.in:1-14,
  * attn_coop.comp.in:1-9).  q: [B, H, Sq, D], k, v: [B, H, Sk, D] views given by (batch, head, seq)

@@ -1,0 +1,145 @@
+"""Matrix-core products at the edges of their tiles: sizes that leave part of a tile or of a 64-element K step,
+every operand layout, K split over partial products, and the int8 linear at such sizes, against float64.
+
+Every operand is a window of a NaN-filled buffer (rows padded to a multiple of 8 elements, as the direct-to-LDS
+kernel needs), so a value read past an edge and not masked turns results into NaN.  Tolerance: the products
+of 16-bit values are exact in fp32 and summed in fp32 (relative error of the sum below 2^-24 sqrt(K) of the
+terms' size, under 1e-5 here), then rounded once: relative L2 below the output's half unit in the last place,
+2^-9 (bf16) or 2^-12 (f16), plus 1e-5."""
+
+import ctypes
+import os
+
+import pytest
+import torch
+
+import torch_vulkan
+from torch_vulkan import abi
+
+dev = torch.device("vk")
+gpu = pytest.mark.gpu
+REL = {torch.bfloat16: 2.0**-9 + 1e-5, torch.float16: 2.0**-12 + 1e-5}
+
+
+def window(rows, cols, dt, gen, transposed):
+    """A [rows, cols] operand on vk inside NaNs, stored row-major or transposed, and its values."""
+    v = torch.randn((rows, cols), generator=gen).to(dt)
+    r, c = (cols, rows) if transposed else (rows, cols)
+    host = torch.full((r + 3, (c + 7) // 8 * 8 + 16), float("nan"), dtype=dt)
+    host[1 : 1 + r, 8 : 8 + c] = v.t() if transposed else v
+    d = host.to(dev)[1 : 1 + r, 8 : 8 + c]
+    return (d.t() if transposed else d), v
+
+
+def check(out, ref, dt):
+    o = out.detach().cpu().double()
+    assert torch.isfinite(o).all()
+    assert ((o - ref).norm() / ref.norm()).item() <= REL[dt]
+
+
+# (M, N, K): one past / one short of the 64-, 128- and 256-wide tiles, K steps with 8 or 56 elements in the partial
+# one, K below one step; the last ones are split along K
+EDGES = [(65, 72, 72), (127, 136, 120), (129, 264, 64), (257, 248, 136), (200, 1000, 40), (600, 520, 1096), (2000, 1304, 264),
+         (4020, 2048, 328), (120, 640, 2936), (24, 72, 4168), (604, 704, 5192)]
+
+
+@gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("m,n,k", EDGES)
+def test_ragged_products(m, n, k, ta, tb, dt):
+    if ta:
+        m = (m + 7) // 8 * 8  # a whole number of 16-byte chunks along the contiguous axis
+    g = torch.Generator().manual_seed(m + n + k)
+    A, a = window(m, k, dt, g, ta)
+    B, b = window(k, n, dt, g, tb)
+    bias = torch.randn((n,), generator=g).to(dt)
+    ref = a.double() @ b.double()
+    check(torch.mm(A, B), ref, dt)
+    out = torch.addmm(bias.to(dev), A, B, alpha=0.5, beta=2.0)
+    check(out, 0.5 * ref + 2.0 * bias.double(), dt)
+    assert torch.equal(out.cpu(), torch.addmm(bias.to(dev), A, B, alpha=0.5, beta=2.0).cpu())
+
+
+@gpu
+@pytest.mark.parametrize("m,n,k", [(777, 943, 64), (65, 129, 200), (1000, 333, 2048), (33, 17, 4096)])
+def test_output_rows_off_16_byte_lines(m, n, k):
+    """N is no multiple of 8 (x W^T): rows of C start at any 2-byte offset."""
+    dt = torch.bfloat16
+    g = torch.Generator().manual_seed(n)
+    A, a = window(m, k, dt, g, False)
+    B, b = window(k, n, dt, g, True)
+    bias = torch.randn((m, n), generator=g).to(dt)
+    check(torch.addmm(bias.to(dev), A, B), a.double() @ b.double() + bias.double(), dt)
+
+
+@gpu
+@pytest.mark.parametrize("ta,tb", [(True, False), (True, True), (False, False)])
+@pytest.mark.parametrize("k", [1, 77, 1001])
+def test_odd_reduction_of_m_and_n_contiguous_operands(k, ta, tb):
+    """K need not be a multiple of 8 where both operands are contiguous along M and N (g^T x over any number of
+    tokens); the other layouts at odd K take the general kernel."""
+    dt = torch.bfloat16
+    g = torch.Generator().manual_seed(k)
+    A, a = window(264, k, dt, g, ta)
+    B, b = window(k, 328, dt, g, tb)
+    check(torch.mm(A, B), a.double() @ b.double(), dt)
+
+
+@gpu
+@pytest.mark.parametrize("m,n,k", [(130, 136, 72), (257, 264, 136)])
+def test_ragged_batches(m, n, k):
+    dt = torch.float16
+    g = torch.Generator().manual_seed(m)
+    a, b = torch.randn((3, m, k), generator=g).to(dt), torch.randn((3, k, n), generator=g).to(dt)
+    check(torch.bmm(a.to(dev), b.to(dev)), torch.bmm(a.double(), b.double()), dt)
+
+
+@gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(1, 200, 320), (17, 72, 2048), (65, 328, 1088), (300, 2000, 512), (1000, 520, 1024),
+                                   (2049, 264, 320)])
+def test_int8_linear_at_ragged_sizes(m, n, k, dt):
+    g = torch.Generator().manual_seed(m + n)
+    X, x = window(m, k, dt, g, False)
+    q = torch.randint(-127, 128, (n, k), generator=g, dtype=torch.int8)
+    s = (torch.rand((n, k // 64), generator=g) * 0.02 + 1e-4).to(torch.bfloat16)
+    bias = torch.randn((n,), generator=g).to(dt)
+    w = (q.double() * s.double().repeat_interleave(64, 1)).to(dt).double()
+    y = torch_vulkan.dequant_int8_linear(X, q.to(dev), s.to(dev), bias.to(dev))
+    check(y, x.double() @ w.t() + bias.double(), dt)
+
+
+@gpu
+def test_infinities_and_nans_stay_in_their_rows():
+    """A ragged product's masked K elements and rows are zeros: an inf or NaN of the operands reaches exactly the
+    outputs whose row or column holds it."""
+    a, b = torch.randn((70, 72)), torch.randn((72, 136))
+    a[3, 71], b[5, 9] = float("inf"), float("nan")
+    a, b = a.bfloat16(), b.bfloat16()
+    out = torch.mm(a.to(dev), b.to(dev)).cpu()
+    ref = (a.double() @ b.double())
+    assert torch.equal(torch.isnan(out), torch.isnan(ref)) and torch.equal(torch.isinf(out), torch.isinf(ref))
+
+
+def plan(m, n, k, a_off=0, **kw):
+    lib = ctypes.CDLL(abi._LIB_PATH)
+    lib.hrt_mm_workspace.restype = ctypes.c_int64
+    lib.hrt_mm_workspace.argtypes = [ctypes.c_void_p]
+    p = abi.MmArgs(a=4096 + a_off, b=8192, c=1 << 20, M=m, N=n, K=k, batch=1, a_sm=k, a_sk=1, b_sk=1, b_sn=k, c_sm=n, c_sn=1)
+    for name, v in kw.items():
+        setattr(p, name, v)
+    return lib.hrt_mm_workspace(ctypes.byref(p))
+
+
+def test_split_plan_on_the_host():
+    """hrt_mm_workspace: whole numbers of [M, N] slices, none for full grids and products with kernels of their own,
+    -1 for operands off 16-byte lines."""
+    assert os.path.exists(abi._LIB_PATH)
+    for m, n, k in [(604, 704, 5184), (300, 64, 4096), (1024, 2048, 8192), (113, 632, 2936)]:
+        w = plan(m, n, k)
+        assert w > 0 and w % (m * n) == 0 and w // (m * n) <= k // 64 // 4, (m, n, k, w)
+    for m, n, k in [(4096, 4096, 4096), (1024, 8192, 2048), (1024, 1024, 1024), (16, 4096, 4096), (4096, 4096, 32)]:
+        assert plan(m, n, k) == 0
+    assert plan(604, 704, 5184, a_off=2) == -1 and plan(604, 704, 5184, c_sn=2) == -1
+    assert plan(604, 704, 5184, batch=2, a_sb=604 * 5184, b_sb=704 * 5184) == 0

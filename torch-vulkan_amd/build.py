@@ -42,6 +42,8 @@ HRT_SOURCES = [
     "kernels/dq8.hip",
     "kernels/gemm.hip",
     "kernels/gemm_mfma.hip",
+    "kernels/gemm_dma_bf16.hip",
+    "kernels/gemm_dma_f16.hip",
     "kernels/rows.hip",
     "kernels/attn_fwd.hip",
     "kernels/attn_bwd.hip",

@@ -171,6 +171,30 @@ __device__ __forceinline__ void dma_tile_part_rs(__amdgpu_buffer_rsrc_t rs, uint
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, tile + j * 1024, 16, (int)lo.off[i % 4], (int)((uint32_t)(j * RPI) * ss), 0, 0);
 }
 
+// Lane offsets of the IPW copies of one wavefront (instructions j0 .. j0 + IPW - 1 of a tile) where only
+// rows [row_lo, row_hi) and chunks [c_lo, c_hi) of the tile exist: the other lanes get an offset beyond the
+// resource's 2^31 - 1 records, and the buffer's range check returns zeros for them, which the copy writes to LDS
+// (checked on the device), so a ragged edge costs no branch, no extra address arithmetic and no memory access.
+// Offsets of existing rows must stay below 2^31 (the launchers check).
+constexpr uint32_t kNoRow = 0x80000000u;
+template <int NCH, int IPW>
+__device__ __forceinline__ void edge_lane_offsets(uint32_t (&off)[IPW], uint32_t ss, int lane, int j0, int row_lo, int row_hi,
+                                                  int c_lo, int c_hi) {
+  constexpr int RPI = 64 / NCH;
+  const int rsub = lane / NCH, slot = lane % NCH;
+#pragma unroll
+  for (int i = 0; i < IPW; ++i) {
+    const int row = (j0 + i) * RPI + rsub, c = slot ^ tile_swz<NCH>(row);
+    off[i] = row >= row_lo && row < row_hi && c >= c_lo && c < c_hi ? (uint32_t)row * ss + (uint32_t)(c << 4) : kNoRow;
+  }
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t edge_rsrc(const HK_G uint8_t* base) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(base), (short)0, 0x7fffffff, 0x00020000);
+}
+__device__ __forceinline__ void edge_copy(__amdgpu_buffer_rsrc_t rs, HK_L uint8_t* tile, int j, uint32_t off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, tile + j * 1024, 16, (int)off, 0, 0, 0);
+}
+
 // First row of the tile that stage st copies when the sequence has more than one stage (len > ROWS): stage
 // st covers rows [st ROWS, (st + 1) ROWS); the last, ragged stage copies the full window that ends at row
 // len - 1 instead (origin len - ROWS), so no copy reads past the sequence, and its rows below st ROWS

@@ -114,42 +114,27 @@ std::optional<Plan> plan(const at::Tensor& a, const at::Tensor& b, const at::Ten
   return p;
 }
 
-// K-split factor of a matrix-core product (1 = no split; unbatched products only, the slices use the batch
-// dimension; K in whole 64-element steps):
+// K-split factor of the matrix-core products that the runtime's own split ("mm_splitk_*") leaves to the caller
+// (1 = no split; unbatched products only, the slices use the batch dimension; K in whole 64-element steps):
 //  * products with an output side of at most 16 (a rank-16 LoRA's x A^T, g B, g^T h, dh^T x) run on the
 //    narrow-output kernel, one workgroup per 16 rows of the long side P, K split across its wavefronts: S
 //    doubles while the P / 16 workgroups times S stay under 256 and every slice keeps >= 1536 of K.  Only
 //    long reductions over few rows repay the second launch: measured at 1024 rows, K = 8192 takes 9.1 us
 //    at S = 4 against 16.3 unsplit, K = 6144 8.2 against 9.0, but K = 2048 5.8 unsplit against 6.7-7.5.
-//  * other narrow products, one 64-wide output tile across (min(M, N) <= 64: rank-16 LoRA factors): S doubles
-//    while the grid of 64 x 64 tiles stays within one workgroup per CU (256) and every slice keeps >= 128
-//    of K;
-//  * wide products whose 128 x 256 (or 256 x 128) tiles alone give fewer than 192 workgroups (1024 x 2048
-//    outputs: 64), which would otherwise fall to 64 x 64 tiles that copy three times the bytes per flop:
-//    S doubles until S x tiles >= 192, keeping >= 1536 of K per slice; the slices then run on the large
-//    tiles.  The fp32 partials cost a write and a read of S x M x N x 4 bytes (32 MB at 1024 x 2048, S = 4),
-//    which only long slices repay: measured at 1024 x 2048 outputs, S = 4 takes 51-52 us against 58-65 at
-//    K = 8192 and 44 against 47 at K = 6144, but 29.5 against 17-19 at K = 2048 (S = 2 loses everywhere:
-//    128 large tiles are too few).  S stays 1 when no split reaches 192 workgroups.
+//  * other narrow products, one 64-wide output tile across (min(M, N) <= 64), whose operands are not 16-byte
+//    aligned: S doubles while the grid of 64 x 64 tiles stays within one workgroup per CU (256) and every
+//    slice keeps >= 128 of K.
 int64_t k_splits(const Plan& p) {
   if (p.batched || p.K % 64 != 0) return 1;
   int64_t s = 1;
   if (std::min(p.M, p.N) <= 16) {
     const int64_t tiles = ((p.N <= 16 ? p.M : p.N) + 15) / 16;
     while (tiles * s < 256 && p.K % (64 * 2 * s) == 0 && p.K / (2 * s) >= 1536) s *= 2;
-    return s;
-  }
-  if (std::min(p.M, p.N) <= 64) {
+  } else if (std::min(p.M, p.N) <= 64) {
     const int64_t tiles = ((p.M + 63) / 64) * ((p.N + 63) / 64), steps = p.K / 64;
     while (tiles * (2 * s) <= 256 && steps % (2 * s) == 0 && p.K / (2 * s) >= 128) s *= 2;
-    return s;
   }
-  const int64_t wide = (p.M % 128 == 0 && p.N % 256 == 0) ? (p.M / 128) * (p.N / 256) : 0;
-  const int64_t tall = (p.M % 256 == 0 && p.N % 128 == 0) ? (p.M / 256) * (p.N / 128) : 0;
-  const int64_t tiles = std::max(wide, tall);
-  if (tiles == 0 || tiles >= 192) return 1;
-  while (tiles * s < 192 && p.K % (64 * 2 * s) == 0 && p.K / (2 * s) >= 1536) s *= 2;
-  return tiles * s >= 192 ? s : 1;
+  return s;
 }
 
 // The split product: slice s of K goes to batch entry s of the matrix-core kernel, which writes unrounded
@@ -206,13 +191,17 @@ std::optional<at::Tensor> try_product(const at::Tensor& a, const at::Tensor& b, 
   if (!p) return std::nullopt;
   at::Tensor out = p->batched ? at::empty({p->batch, p->M, p->N}, a.options()) : at::empty({p->M, p->N}, a.options());
   const bool matrix_cores = p->dt != at::kFloat && gate().admits(p->batched);
-  const int64_t S = matrix_cores ? k_splits(*p) : 1;
-  if (S > 1) {
-    run_split(*p, S, out);
+  hrt_mm_args A = p->args;
+  A.c = dptr(out);
+  const int64_t ws = matrix_cores && !p->batched ? hrt_mm_workspace(&A) : 0;
+  if (ws > 0) {
+    const at::Tensor partial = at::empty({ws}, out.options().dtype(at::kFloat));
+    const hrt_mm_splitk_args X{A, dptr(partial), ws};
+    queue(typed("mm_splitk", p->dt), X);
   } else {
-    hrt_mm_args A = p->args;
-    A.c = dptr(out);
-    queue(typed(matrix_cores ? "mm_mfma" : "mm", p->dt), A);
+    const int64_t S = matrix_cores && (ws < 0 || std::min(p->M, p->N) <= 16) ? k_splits(*p) : 1;
+    if (S > 1) run_split(*p, S, out);
+    else queue(typed(matrix_cores ? "mm_mfma" : "mm", p->dt), A);
   }
   static const bool verify = std::getenv("VKT_VERIFY_MM") != nullptr;
   if (verify && matrix_cores) verify_with_fma(*p, out);

@@ -40,7 +40,7 @@ at::Tensor dequant_int8_vk(const at::Tensor& q, const at::Tensor& scale, at::Sca
 
 // y = x @ deq(q)^T (+ bias) for x [..., K] bf16/f16, q [N, K]: y [..., N] in x's dtype.  For M >= 2048 rows the
 // weights are dequantized once into a workspace and the product runs on them (the fused kernel would
-// convert each weight once per 256 rows of x); the values are the same either way.
+// convert each weight once per 256 rows of x); for few rows the workspace holds partial products over K.
 at::Tensor dequant_int8_linear_vk(const at::Tensor& x, const at::Tensor& q, const at::Tensor& scale,
                                   const std::optional<at::Tensor>& bias) {
   check_weights(q, scale, "dequant_int8_linear");
@@ -65,7 +65,7 @@ at::Tensor dequant_int8_linear_vk(const at::Tensor& x, const at::Tensor& q, cons
     A.bias = dptr(*bias), A.has_bias = 1;
   }
   at::Tensor deq;
-  if (M >= 2048) {
+  if (hrt_mm_dq8_workspace(&A) > 0) {
     deq = at::empty({N, K}, x.options());
     A.ws = dptr(deq);
   }
