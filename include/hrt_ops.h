@@ -139,7 +139,7 @@ typedef struct hrt_ew_args {
   int64_t c_strides[HRT_MAX_DIMS];
 } hrt_ew_args;
 
-/* "mm_{f32,bf16,f16}" (portable FMA kernel) and "mm_mfma_{bf16,f16}" (gfx950 matrix cores):
+/* "mm_{f32,bf16,f16}" (f32: the fp32 matrix cores; bf16, f16: portable FMA kernel) and "mm_mfma_{bf16,f16}" (gfx950 matrix cores):
  *   c[b, m, n] = alpha * sum_k a[b, m, k] * b[b, k, n] + beta * bias[b, m, n]     (bias only if has_bias)
  * a, b, bias: any non-negative strides (transposed / sliced views are read in place; bias broadcasts
  * with stride 0); c: written with strides c_s*.  fp32 accumulation, one rounding at the store.
@@ -172,9 +172,9 @@ typedef struct hrt_mm_reduce_args {
   uint32_t has_bias, pad;
 } hrt_mm_reduce_args;
 
-/* "mm_splitk_{bf16,f16}" — the product of "mm_mfma_{bf16,f16}" (flags 0) with K split over fp32 partial products
+/* "mm_splitk_{f32,bf16,f16}" — the product of "mm_f32" / "mm_mfma_{bf16,f16}" (flags 0) with K split over fp32 partial products
  * where that is faster, and their ordered sum, in one call (no counterpart in the reference).  ws: at least
- * hrt_mm_workspace(&mm) floats, 16-byte aligned, ws_floats of them; 0 floats: the plain product. */
+ * hrt_mm_workspace(&mm, dtype) floats, 16-byte aligned, ws_floats of them; 0 floats: the plain product. */
 typedef struct hrt_mm_splitk_args {
   hrt_mm_args mm;
   uint64_t ws;
@@ -182,7 +182,7 @@ typedef struct hrt_mm_splitk_args {
 } hrt_mm_splitk_args;
 /* fp32 elements of workspace "mm_splitk_*" uses for this product (0: it is not split; -1: its operands
  * are not aligned as the split kernel needs).  A pure host function of the sizes, strides and alignments. */
-int64_t hrt_mm_workspace(const hrt_mm_args* mm);
+int64_t hrt_mm_workspace(const hrt_mm_args* mm, int32_t dtype);
 
 /* "mm_dq8_{bf16,f16}" — fused int8 weight-only linear (no reference counterpart; composes
  * csrc/ops_quant.cpp:34-59 with csrc/ops_mm.cpp:61-175):

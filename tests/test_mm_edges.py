@@ -110,6 +110,56 @@ def test_int8_linear_at_ragged_sizes(m, n, k, dt):
     check(y, x.double() @ w.t() + bias.double(), dt)
 
 
+# fp32 (fp32 matrix cores): 16-byte and 4-byte copies (odd sizes, offset views), every layout, split K, batches.
+# Tolerance: an fp32 sum of K products, each fused multiply-add rounding to half a unit in the last place of the
+# partial sum: relative L2 below 2^-24 sqrt(K) for random signs, doubled.
+F32_EDGES = [(64, 64, 32), (65, 63, 33), (1, 1, 1), (130, 200, 31), (72, 136, 100), (127, 65, 257), (300, 512, 3001), (128, 128, 4096),
+             (1000, 1000, 64)]
+
+
+@gpu
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("m,n,k", F32_EDGES)
+def test_f32_products(m, n, k, offset, ta, tb):
+    g = torch.Generator().manual_seed(m + n + k)
+
+    def make(rows, cols, transposed):
+        v = torch.randn((rows, cols), generator=g)
+        r, c = (cols, rows) if transposed else (rows, cols)
+        host = torch.full((r + 2, (c + 3) // 4 * 4 + 8), float("nan"))
+        host[1 : 1 + r, 4 + offset : 4 + offset + c] = v.t() if transposed else v
+        d = host.to(dev)[1 : 1 + r, 4 + offset : 4 + offset + c]
+        return (d.t() if transposed else d), v
+
+    A, a = make(m, k, ta)
+    B, b = make(k, n, tb)
+    bias = torch.randn((n,), generator=g)
+    ref = a.double() @ b.double()
+    tol = 2.0**-23 * k**0.5 + 2.0**-23
+    out = torch.mm(A, B).cpu()
+    assert ((out - ref).norm() / ref.norm()).item() <= tol
+    out = torch.addmm(bias.to(dev), A, B, alpha=0.5, beta=2.0).cpu()
+    want = 0.5 * ref + 2.0 * bias.double()
+    assert ((out - want).norm() / want.norm()).item() <= 2 * tol
+
+
+@gpu
+def test_f32_strided_batches_and_small_values():
+    g = torch.Generator().manual_seed(0)
+    a, b = torch.randn((3, 70, 90), generator=g), torch.randn((3, 50, 180), generator=g)
+    A, B = a.to(dev), b.to(dev)[:, :, ::2].transpose(1, 2)  # k strided by 2: no contiguous axis
+    ref = a.double() @ b.double()[:, :, ::2].transpose(1, 2)
+    assert ((torch.bmm(A, B).cpu() - ref).norm() / ref.norm()).item() <= 2.0**-23 * 90**0.5
+    x, y = torch.full((64, 64), 1e-30), torch.full((64, 64), 1e-10)  # subnormal products are kept
+    z = torch.mm(x.to(dev), y.to(dev)).cpu().double()
+    assert torch.allclose(z, torch.full_like(z, 64e-40), rtol=1e-4)
+    inf = torch.zeros((64, 64))
+    inf[3, 5] = float("inf")
+    o = torch.mm(inf.to(dev), torch.ones((64, 64)).to(dev)).cpu()
+    assert torch.isinf(o[3]).all() and torch.equal(o[:3], torch.zeros(3, 64)) and torch.isfinite(o[4:]).all()
+
+
 @gpu
 def test_infinities_and_nans_stay_in_their_rows():
     """A ragged product's masked K elements and rows are zeros: an inf or NaN of the operands reaches exactly the
@@ -122,14 +172,14 @@ def test_infinities_and_nans_stay_in_their_rows():
     assert torch.equal(torch.isnan(out), torch.isnan(ref)) and torch.equal(torch.isinf(out), torch.isinf(ref))
 
 
-def plan(m, n, k, a_off=0, **kw):
+def plan(m, n, k, a_off=0, dtype=abi.BF16, **kw):
     lib = ctypes.CDLL(abi._LIB_PATH)
     lib.hrt_mm_workspace.restype = ctypes.c_int64
-    lib.hrt_mm_workspace.argtypes = [ctypes.c_void_p]
+    lib.hrt_mm_workspace.argtypes = [ctypes.c_void_p, ctypes.c_int32]
     p = abi.MmArgs(a=4096 + a_off, b=8192, c=1 << 20, M=m, N=n, K=k, batch=1, a_sm=k, a_sk=1, b_sk=1, b_sn=k, c_sm=n, c_sn=1)
     for name, v in kw.items():
         setattr(p, name, v)
-    return lib.hrt_mm_workspace(ctypes.byref(p))
+    return lib.hrt_mm_workspace(ctypes.byref(p), dtype)
 
 
 def test_split_plan_on_the_host():
@@ -142,4 +192,6 @@ def test_split_plan_on_the_host():
     for m, n, k in [(4096, 4096, 4096), (1024, 8192, 2048), (1024, 1024, 1024), (16, 4096, 4096), (4096, 4096, 32)]:
         assert plan(m, n, k) == 0
     assert plan(604, 704, 5184, a_off=2) == -1 and plan(604, 704, 5184, c_sn=2) == -1
+    assert plan(128, 128, 4096, dtype=abi.F32) % (128 * 128) == 0 and plan(128, 128, 4096, dtype=abi.F32) > 0
+    assert plan(2048, 2048, 64, dtype=abi.F32) == 0
     assert plan(604, 704, 5184, batch=2, a_sb=604 * 5184, b_sb=704 * 5184) == 0

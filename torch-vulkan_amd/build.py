@@ -41,6 +41,7 @@ HRT_SOURCES = [
     "kernels/conv3x3.hip",
     "kernels/dq8.hip",
     "kernels/gemm.hip",
+    "kernels/gemm_f32.hip",
     "kernels/gemm_mfma.hip",
     "kernels/gemm_dma_bf16.hip",
     "kernels/gemm_dma_f16.hip",

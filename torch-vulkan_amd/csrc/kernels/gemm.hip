@@ -1,12 +1,17 @@
 // Portable GEMM "mm_{f32,bf16,f16}": c = alpha * a @ b + beta * bias with arbitrary strides, fp32 FMA.
-// Serves the f32 path (where fp32 accuracy is required) and bf16/f16 when matrix cores are switched off,
+// Serves bf16/f16 when the matrix cores are switched off and the f32 products that gemm_f32.hip does not take,
 // like the reference's tiled kernel vkrt/shaders/mm.comp.in:90-154 (same math: fp32 accumulate, epilogue
 // alpha*acc + beta*bias, one rounding at the store).  64x64 output tile per 256-thread workgroup, 4x4 per
 // thread, K in steps of 16 staged through LDS as fp32.
+#include <type_traits>
+
 #include "../hrt/registry.h"
 #include "device_common.h"
 
 namespace hk {
+
+bool mm_f32_mfma(const hrt_mm_args& a, hipStream_t s);  // gemm_f32.hip
+
 namespace {
 
 constexpr int BM = 64, BN = 64, BK = 16;
@@ -108,6 +113,8 @@ bool launch_mm_fma(const void* p, const uint32_t*, hrt::LaunchCtx& ctx) {
   const auto& a = *static_cast<const hrt_mm_args*>(p);
   if (a.flags != 0) return ctx.fail("the FMA GEMM takes no flags");
   if (!mm_check_operands(a, sizeof(typename T::storage), ctx)) return false;
+  if constexpr (std::is_same<T, F32>::value)  // the fp32 matrix cores, unless its 31-bit offsets do not reach
+    if (mm_f32_mfma(a, ctx.stream)) return hrt::launch_ok(hipGetLastError(), ctx, "mm_f32_dma");
   if (cdiv(a.M, BM) > 65535) return ctx.fail("M too large for the FMA kernel grid");
   const dim3 grid((uint32_t)cdiv(a.N, BN), (uint32_t)cdiv(a.M, BM), (uint32_t)a.batch);
   hipLaunchKernelGGL(mm_fma<T>, grid, dim3(256), 0, ctx.stream, a);

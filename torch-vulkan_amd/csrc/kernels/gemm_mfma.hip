@@ -16,6 +16,7 @@
 //     gives each XCD a band of N-panels that it reads once into its own L2.
 // This general kernel takes what the direct-to-LDS kernel (gemm_dma_kernel.h) does not: operand rows off 16-byte
 // lines, a strided C.  The choice between them, the tile and the K split are made here (plan_gemm).
+#include <array>
 #include <cstring>
 #include <type_traits>
 #include <utility>
@@ -28,6 +29,7 @@
 namespace hk {
 
 bool mm_check_operands(const hrt_mm_args& a, uint64_t elem, hrt::LaunchCtx& ctx);
+int64_t mm_f32_workspace(const hrt_mm_args& a);  // gemm_f32.hip
 
 namespace {
 
@@ -380,12 +382,14 @@ struct GemmPlan {
 
 // The cheapest tile, and for one product (no batch) the cheapest number of K slices when may_split: under-filled
 // grids with a long reduction then run several slices per tile, whose fp32 partial products a second kernel adds
-// in order.  A split has to promise 5% more than an unsplit tile.
-GemmPlan plan_gemm(const hrt_mm_args& a, bool may_split) {
-  GemmPlan best;
+// in order.  A split has to promise 8 us: its workspace and second launch cost the host 4 us, which a program of small
+// layers waits for.
+GemmPlan search_plan(const hrt_mm_args& a, bool may_split) {
+  GemmPlan best, whole;
   const bool f32out = (a.flags & HRT_MM_F32_OUT) != 0;
   const int64_t nk = cdiv(a.K, GBK);
   double best_us = 0.0;
+  double whole_us = 0.0;
   static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
   for (int t = 0; t < kGemmTiles; ++t) {
     const DmaForm f = dma_form(a, kTileShape[t].bm, kTileShape[t].bn);
@@ -402,11 +406,26 @@ GemmPlan plan_gemm(const hrt_mm_args& a, bool may_split) {
       if (s > 1 && (!may_split || !slices_ok || a.batch != 1 || nk < 4 * s || tiles * s > 2 * kTileCost[t].slots)) break;
       const uint32_t per = (uint32_t)(nk + s - 1) / s, n = ((uint32_t)nk + per - 1) / per;
       double us = (lines ? 1.25 : 1.0) * tile_us(kTileCost[t], kTileShape[t], tiles * n, per);
-      if (n > 1) us = 1.05 * (us + split_us(n, a.M, a.N));
-      if (best.tile < 0 || us < best_us) best_us = us, best = GemmPlan{t, n, n > 1 ? per * GBK : 0};
+      if (n > 1) us += split_us(n, a.M, a.N);
+      const GemmPlan p{t, n, n > 1 ? (int64_t)per * GBK : 0};
+      if (n == 1 && (whole.tile < 0 || us < whole_us)) whole_us = us, whole = p;
+      if (best.tile < 0 || us < best_us) best_us = us, best = p;
     }
   }
-  return best;
+  return best.splits > 1 && whole.tile >= 0 && best_us > whole_us - 8.0 ? whole : best;
+}
+
+// The shim asks for a workspace and then queues the same product: the last plan is kept, by the values it depends on
+// (an unsplit choice among splits is the choice without them too).
+GemmPlan plan_gemm(const hrt_mm_args& a, bool may_split) {
+  const std::array<int64_t, 17> key = {a.M, a.N, a.K, a.batch, a.a_sb, a.a_sm, a.a_sk, a.b_sb, a.b_sk, a.b_sn, a.c_sb, a.c_sm, a.c_sn,
+                                       (int64_t)(a.a % 16), (int64_t)(a.b % 16), (int64_t)(a.c % 16), (int64_t)a.flags};
+  thread_local std::array<int64_t, 17> last_key{};  // M = 0: no plan yet
+  thread_local GemmPlan last;
+  thread_local bool last_split = false;
+  if (key != last_key || (may_split != last_split && !(last_split && last.splits == 1)))
+    last = search_plan(a, may_split), last_key = key, last_split = may_split;
+  return last;
 }
 
 // Which loader an operand can use.  rows = M (A) or N (B); s_r / s_k its strides.
@@ -731,8 +750,10 @@ hrt_mm_args dq8_as_mm(const hrt_mm_dq8_args& d) {
 
 }  // namespace hk
 
-extern "C" int64_t hrt_mm_workspace(const hrt_mm_args* a) {
-  if (a == nullptr || a->M <= 0 || a->N <= 0 || a->K <= 0 || a->batch != 1 || a->flags != 0 || hk::own_kernel(*a)) return 0;
+extern "C" int64_t hrt_mm_workspace(const hrt_mm_args* a, int32_t dtype) {
+  if (a == nullptr || a->M <= 0 || a->N <= 0 || a->K <= 0 || a->batch != 1 || a->flags != 0) return 0;
+  if (dtype == HRT_F32) return hk::mm_f32_workspace(*a);
+  if ((dtype != HRT_BF16 && dtype != HRT_F16) || hk::own_kernel(*a)) return 0;
   const hk::GemmPlan p = hk::plan_gemm(*a, true);
   return p.tile < 0 ? -1 : p.splits > 1 ? p.splits * a->M * a->N : 0;
 }

@@ -6,9 +6,9 @@
 // A call is planned as one product C[b] = alpha * A[b] @ B[b] + beta * bias[b] over [batch, M, N, K]:
 // operands are described by their element strides (transposed and sliced views cost nothing), the bias by
 // the strides of its broadcast to the output shape (PyTorch's own expand).  The plan then goes to one of
-// three engines: the gfx950 matrix-core kernel "mm_mfma_*" (bf16/f16), the same kernel over split K
-// ranges plus the ordered reduction "mm_reduce_*" (products one 64-wide tile across, e.g. rank-16 LoRA
-// factors), or the FMA kernel "mm_*" (f32, and bf16/f16 when the matrix cores are switched off).
+// three engines: the gfx950 matrix-core kernels "mm_mfma_*" (bf16/f16) and "mm_f32", the same kernels over
+// split K ranges plus an ordered sum ("mm_splitk_*" where the runtime plans the split, else "mm_reduce_*": rank-16
+// LoRA factors), or the FMA kernels "mm_{bf16,f16}" when the matrix cores are switched off.
 //
 // Debug aids: set_coop_range / VKT_NO_COOP (the matrix-core gate below) and VKT_VERIFY_MM=1, which
 // recomputes every matrix-core product with the FMA kernel and reports calls whose results disagree.
@@ -193,7 +193,7 @@ std::optional<at::Tensor> try_product(const at::Tensor& a, const at::Tensor& b, 
   const bool matrix_cores = p->dt != at::kFloat && gate().admits(p->batched);
   hrt_mm_args A = p->args;
   A.c = dptr(out);
-  const int64_t ws = matrix_cores && !p->batched ? hrt_mm_workspace(&A) : 0;
+  const int64_t ws = (matrix_cores || p->dt == at::kFloat) && !p->batched ? hrt_mm_workspace(&A, float_code(p->dt)) : 0;
   if (ws > 0) {
     const at::Tensor partial = at::empty({ws}, out.options().dtype(at::kFloat));
     const hrt_mm_splitk_args X{A, dptr(partial), ws};
