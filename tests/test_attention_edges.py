@@ -1,0 +1,72 @@
+"""Fused attention at the edges of its kernels' tiles, against float64: several streamed stages with a partial last
+one, head dimensions at and off the tile widths, row strides and alignments, few keys under many queries.
+
+Operands are windows of NaN-filled buffers, so a value read past an edge and not masked shows.  Tolerance (relative L2
+of o, dq, dk, dv): f32 the accumulation of D and S products and two exponentials' rounding, 2^-24 (sqrt(D) + sqrt(S) +
+16) with a factor 2; bf16 / f16 the bounds that the other attention tests use."""
+
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+import torch_vulkan
+
+pytestmark = pytest.mark.gpu
+dev = torch.device("vk")
+REL16 = {torch.bfloat16: 1e-2, torch.float16: 4e-3}
+
+
+@pytest.fixture(autouse=True)
+def _always_fused():
+    torch_vulkan.set_fused_attention("on")
+    yield
+    torch_vulkan.set_fused_attention("auto")
+
+
+def operand(B, S, H, D, dt, g, pad, offset):
+    """[B, H, S, D] view of token-major memory with NaN rows and columns around it."""
+    v = torch.randn((B, S, H, D), generator=g).to(dt)
+    host = torch.full((B, S + 1, H, D + pad), float("nan"), dtype=dt)
+    host[:, :S, :, offset : offset + D] = v
+    return host.to(dev)[:, :S, :, offset : offset + D].transpose(1, 2).detach().requires_grad_(True), v.double().transpose(1, 2)
+
+
+def check(B, H, Sq, Sk, D, dt, rel, pad=8, offset=0):
+    g = torch.Generator().manual_seed(Sq + Sk + D)
+    (q, q64), (k, k64), (v, v64) = (operand(B, s, H, D, dt, g, pad, offset) for s in (Sq, Sk, Sk))
+    go = torch.randn((B, H, Sq, D), generator=g).to(dt)
+    out = F.scaled_dot_product_attention(q, k, v)
+    got = (out,) + torch.autograd.grad(out, (q, k, v), go.to(dev))
+    leaves = [t.clone().requires_grad_(True) for t in (q64, k64, v64)]
+    ref = torch.softmax(leaves[0] @ leaves[1].transpose(-1, -2) / math.sqrt(D), -1) @ leaves[2]
+    want = (ref,) + torch.autograd.grad(ref, leaves, go.double())
+    for name, a, b in zip(("o", "dq", "dk", "dv"), got, want):
+        a = a.detach().cpu().double()
+        assert torch.isfinite(a).all(), name
+        e = ((a - b).norm() / b.norm()).item()
+        assert e <= rel, (name, e)
+    again = F.scaled_dot_product_attention(q, k, v)
+    rep = (again,) + torch.autograd.grad(again, (q, k, v), go.to(dev))
+    assert all(torch.equal(a.detach().cpu(), b.detach().cpu()) for a, b in zip(got, rep))  # same bits twice
+
+
+def f32_rel(Sk, D):
+    return 2 * 2.0**-24 * (math.sqrt(D) + math.sqrt(Sk) + 16)
+
+
+@pytest.mark.parametrize("D", [8, 30, 32, 40, 64, 68, 96, 112, 128])
+@pytest.mark.parametrize("Sq,Sk", [(333, 777), (129, 64), (64, 129), (260, 31)])
+def test_f32_stages_and_head_dims(Sq, Sk, D):
+    check(2, 3, Sq, Sk, D, torch.float32, f32_rel(max(Sq, Sk), D))
+
+
+@pytest.mark.parametrize("D,pad,offset", [(64, 4, 4), (64, 3, 1), (128, 5, 2), (33, 4, 0)])
+def test_f32_strides_and_alignments(D, pad, offset):
+    check(1, 2, 200, 300, D, torch.float32, f32_rel(300, D), pad, offset)
+
+
+def test_f32_many_workgroups():
+    """More workgroups than the chip holds at once, a partial last stage."""
+    check(1, 16, 1050, 1050, 64, torch.float32, f32_rel(1050, 64))

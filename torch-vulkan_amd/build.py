@@ -49,6 +49,7 @@ HRT_SOURCES = [
     "kernels/attn_fwd.hip",
     "kernels/attn_bwd.hip",
     "kernels/attn_f32.hip",
+    "kernels/attn_f32_mfma.hip",
 ]
 SHIM_SOURCES = [
     "shim/device.cpp",

@@ -1,11 +1,12 @@
 // Fused attention with fp32 arithmetic throughout: "attn_{fwd,dkdv,dq}_fma_{f32,bf16,f16}".
 //
-// The f32 path of the reference (vkrt/shaders/attn.comp.in:256-395, its scalar kernels) and the bf16/f16
-// path when matrix cores are switched off: logits, P and dS stay fp32 (no rounding before the second
+// The bf16/f16 path when matrix cores are switched off, and the f32 calls whose row strides attn_f32_mfma.hip does not
+// take (the reference's scalar kernels, vkrt/shaders/attn.comp.in:256-395): logits, P and dS stay fp32 (no rounding before the second
 // products), so f32 inputs meet a 1e-5 relative L2 bound.  Not the performance path: one wavefront of
 // 64 lanes per workgroup, one query (forward, dQ) or key (dK/dV) per lane, the streamed operand staged in
 // LDS as fp32 and read as broadcasts, the lane's own rows kept in LDS with a +1 padded stride.
 #include <cmath>
+#include <type_traits>
 
 #include "../hrt/registry.h"
 #include "device_common.h"
@@ -13,6 +14,7 @@
 namespace hk {
 
 bool attn_check(const hrt_attn_args& a, bool fwd, bool dkdv, bool dq, uint64_t elem, hrt::LaunchCtx& ctx);
+bool attn_f32_mfma(const hrt_attn_args& a, int which, hipStream_t s);  // attn_f32_mfma.hip
 
 namespace {
 
@@ -214,6 +216,8 @@ bool launch_fma(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   const int nb = ((W == 1 ? a.Sk : a.Sq) + 63) / 64;
   const int64_t total = (int64_t)nb * a.B * a.H;
   if (total > 0x7fffffffLL) return ctx.fail("grid too large");
+  if constexpr (std::is_same<T, F32>::value)  // the fp32 matrix cores, unless their 31-bit offsets do not reach
+    if (attn_f32_mfma(a, W, ctx.stream)) return hrt::launch_ok(hipGetLastError(), ctx, "attn_f32_mfma");
   const dim3 g((uint32_t)total);
   const int dch = (a.D + 31) / 32;
 #define HK_ATTN_FMA(DPV)                                                                         \
