@@ -230,6 +230,9 @@ int64_t hrt_mm_dq8_workspace(const hrt_mm_dq8_args* args);
  * in the reference: PyTorch's autograd copies a leaf's gradient into the leaf's own layout, so gradients
  * in the input's layout cost nothing there; the caller must give q, k, v non-overlapping dense layouts. */
 #define HRT_ATTN_GRAD_LIKE_INPUT 4u
+/* "attn_dkdv_{bf16,f16}" with this flag: o32 is hrt_attn_dkdv_workspace(&args) floats of workspace, 16-byte aligned.
+ * No counterpart in the reference. */
+#define HRT_ATTN_DKDV_WS 8u
 typedef struct hrt_attn_args {
   uint64_t q, k, v;
   uint64_t o, lse, o32;
@@ -243,6 +246,10 @@ typedef struct hrt_attn_args {
   float scale;
   uint32_t flags, pad;
 } hrt_attn_args;
+/* fp32 elements of workspace with which "attn_dkdv_{bf16,f16}" (matrix-core kernels) is faster, 0 when it has no use
+ * for one: with few key blocks the queries of a block are then shared out over workgroups, whose partial dK, dV are
+ * added in order (HRT_ATTN_DKDV_WS). */
+int64_t hrt_attn_dkdv_workspace(const hrt_attn_args* args);
 
 /* Row softmax over R of a contiguous [outer, R, inner] tensor (vkrt/shaders/softmax.comp.in:27-50):
  *  "softmax_fwd_{dt}": y = exp(x - max) / sum(exp(x - max)); with safe != 0 a row whose entries are all

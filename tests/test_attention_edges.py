@@ -70,3 +70,24 @@ def test_f32_strides_and_alignments(D, pad, offset):
 def test_f32_many_workgroups():
     """More workgroups than the chip holds at once, a partial last stage."""
     check(1, 16, 1050, 1050, 64, torch.float32, f32_rel(1050, 64))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [40, 48, 56, 72, 80, 96, 104, 120, 36])
+@pytest.mark.parametrize("Sq,Sk", [(333, 333), (64, 300), (129, 77), (520, 130)])
+def test_16_bit_head_dims_between_the_tile_widths(Sq, Sk, D, dt):
+    """D % 8 == 0: the direct-to-LDS kernels with masked columns; 36: the general kernel."""
+    check(1, 3, Sq, Sk, D, dt, REL16[dt])
+
+
+@pytest.mark.parametrize("D", [40, 64, 80, 128])
+@pytest.mark.parametrize("B,H,Sq,Sk", [(1, 4, 1024, 77), (2, 3, 2048, 8), (1, 2, 1000, 200), (1, 1, 700, 64), (1, 8, 640, 513), (1, 1, 513, 2)])
+def test_few_keys_share_out_the_queries(B, H, Sq, Sk, D):
+    """dK / dV of few key blocks: the query stages (whole and partial last) go to several workgroups per block.
+    (With one key dq and dk are exactly 0 and have no relative error; two keys is the smallest case here.)"""
+    check(B, H, Sq, Sk, D, torch.float16, REL16[torch.float16])
+
+
+@pytest.mark.parametrize("pad,offset", [(8, 8), (4, 4), (5, 3)])
+def test_16_bit_alignments(pad, offset):
+    check(1, 2, 300, 200, 80, torch.float16, REL16[torch.float16], pad, offset)

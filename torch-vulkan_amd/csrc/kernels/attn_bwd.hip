@@ -401,7 +401,7 @@ __global__ __launch_bounds__(256) void attn_dq_mfma(hrt_attn_args p, int nqb) {
   }
 }
 
-// ---- dQ fast path: D = 64 or 128, 16-byte aligned rows ------------------------------------------------------
+// ---- dQ fast path: D a multiple of 8 above 32, 16-byte aligned rows ------------------------------------------------------
 //
 // The forward kernel's structure applied to dQ: K and V stages (128 keys) go global -> LDS directly and
 // double-buffered; 8 wavefronts, wave (g = w & 1, k = w >> 1) handles query group g (32 rows of the 64-row
@@ -414,7 +414,8 @@ __global__ __launch_bounds__(256) void attn_dq_mfma(hrt_attn_args p, int nqb) {
 // quarter, summed through LDS, vkrt/shaders/attn.comp.in:210-240) and stores it for the dK/dV kernel.
 constexpr int KST2 = 128;  // keys per LDS stage
 
-template <typename T, int DCH, bool OF32, bool WITH_DELTA>
+// PAD: as the forward's (columns D and up are zeros in LDS, not stored).
+template <typename T, int DCH, bool OF32, bool WITH_DELTA, bool PAD>
 __global__ __launch_bounds__(512) void attn_dq_dma(hrt_attn_args p, int nqb) {
   constexpr int NW = 8;
   constexpr int NCH = DCH * 4;
@@ -445,7 +446,9 @@ __global__ __launch_bounds__(512) void attn_dq_dma(hrt_attn_args p, int nqb) {
   const int nst = (Sk + KST2 - 1) / KST2;
 
   const int j0 = wave * (KST2 * NCH / 64 / NW);
-  const DmaLanes klo = dma_lane_offsets<NCH>(kss, lane, j0), vlo = dma_lane_offsets<NCH>(vss, lane, j0);
+  const int dch = PAD ? p.D / 8 : NCH;  // chunks of a row that exist
+  const DmaLanes klo = PAD ? edge_lanes<NCH>(kss, lane, j0, dch) : dma_lane_offsets<NCH>(kss, lane, j0);
+  const DmaLanes vlo = PAD ? edge_lanes<NCH>(vss, lane, j0, dch) : dma_lane_offsets<NCH>(vss, lane, j0);
   // The block's 64 rows of Q and dO go to the stage-1 buffers (free until stage 0 copies into them), copied
   // once for the four wavefronts that share them, ahead of K(0), V(0); rows past Sq hold copies of the last
   // row (P = 0 for them: lse = -inf below)
@@ -457,8 +460,13 @@ __global__ __launch_bounds__(512) void attn_dq_dma(hrt_attn_args p, int nqb) {
                                qb * 64 * (int64_t)qss;
     const HK_G uint8_t* Oblk = reinterpret_cast<const HK_G uint8_t*>(gcptr<uint16_t>(p.dout) + b * p.do_sb + hh * p.do_sh) +
                                qb * 64 * (int64_t)oss;
-    dma_tile<NCH, 64, NW>(Qblk, qss, qvalid, K1, wave, lane, dma_lane_offsets<NCH>(qss, lane, jq));
-    dma_tile<NCH, 64, NW>(Oblk, oss, qvalid, V1, wave, lane, dma_lane_offsets<NCH>(oss, lane, jq));
+    if constexpr (PAD) {
+      edge_tile<NCH, 64, NW>(Qblk, qss, qvalid, dch, K1, wave, lane);
+      edge_tile<NCH, 64, NW>(Oblk, oss, qvalid, dch, V1, wave, lane);
+    } else {
+      dma_tile<NCH, 64, NW>(Qblk, qss, qvalid, K1, wave, lane, dma_lane_offsets<NCH>(qss, lane, jq));
+      dma_tile<NCH, 64, NW>(Oblk, oss, qvalid, V1, wave, lane, dma_lane_offsets<NCH>(oss, lane, jq));
+    }
   }
 
   const int64_t q = qb * 64 + g * 32 + ql;
@@ -473,6 +481,11 @@ __global__ __launch_bounds__(512) void attn_dq_dma(hrt_attn_args p, int nqb) {
 #pragma unroll
     for (int i = 0; i < KSQ; ++i) {
       const int d0 = (kq * KSQ + i) * 16 + 8 * hl;
+      if (PAD && d0 >= p.D) {  // no such columns: their dO is zero, o has to be finite
+#pragma unroll
+        for (int w = 0; w < OV; ++w) oraw[OV * i + w] = u32x4{0, 0, 0, 0};
+        continue;
+      }
       if constexpr (OF32) {
         oraw[2 * i] = *reinterpret_cast<const HK_G u32x4*>(gcptr<float>(p.o) + orow + d0);
         oraw[2 * i + 1] = *reinterpret_cast<const HK_G u32x4*>(gcptr<float>(p.o) + orow + d0 + 4);
@@ -484,8 +497,13 @@ __global__ __launch_bounds__(512) void attn_dq_dma(hrt_attn_args p, int nqb) {
   float dlt = 0.f;
   if constexpr (!WITH_DELTA) dlt = gcptr<float>(p.delta)[bh * Sq + (qv ? q : 0)];
   issue_order_fence();  // the first barrier counts on K(0), V(0) being the last copies issued
-  dma_tile<NCH, KST2, NW>(Kb, kss, Sk, K0, wave, lane, klo);
-  dma_tile<NCH, KST2, NW>(Vb, vss, Sk, V0, wave, lane, vlo);
+  if constexpr (PAD) {
+    edge_tile<NCH, KST2, NW>(Kb, kss, Sk, dch, K0, wave, lane);
+    edge_tile<NCH, KST2, NW>(Vb, vss, Sk, dch, V0, wave, lane);
+  } else {
+    dma_tile<NCH, KST2, NW>(Kb, kss, Sk, K0, wave, lane, klo);
+    dma_tile<NCH, KST2, NW>(Vb, vss, Sk, V0, wave, lane, vlo);
+  }
 
   int koff[2 * DCH], voff[DCH][2];
 #pragma unroll
@@ -540,7 +558,7 @@ __global__ __launch_bounds__(512) void attn_dq_dma(hrt_attn_args p, int nqb) {
     part = halfswap_sum(qv ? part : 0.f);
     if (hl == 0) xdel[kq][g * 32 + ql] = part;
   }
-  __syncthreads();  // stage 0 in LDS; partial deltas published; Q / dO read out of the stage-1 buffers
+  barrier_keep_vm_lds<0>();  // stage 0 in LDS; partial deltas published; Q / dO read out of the stage-1 buffers
   if constexpr (WITH_DELTA) {
     dlt = xdel[0][g * 32 + ql] + xdel[1][g * 32 + ql] + xdel[2][g * 32 + ql] + xdel[3][g * 32 + ql];
     if (kq == 0 && hl == 0 && qv) gptr<float>(p.delta)[bh * Sq + q] = dlt;
@@ -557,8 +575,9 @@ __global__ __launch_bounds__(512) void attn_dq_dma(hrt_attn_args p, int nqb) {
     constexpr bool COPY = decltype(cc)::value;
     const int64_t key0 = (int64_t)st * KST2;
     // buffer resources over the next stage's first rows (scalar row offsets, no 64-bit address arithmetic)
-    const __amdgpu_buffer_rsrc_t krs = dma_rsrc(Kb + stage_origin<KST2>(st + 1, nst, Sk) * kss);
-    const __amdgpu_buffer_rsrc_t vrs = dma_rsrc(Vb + stage_origin<KST2>(st + 1, nst, Sk) * vss);
+    const HK_G uint8_t* const kn = Kb + stage_origin<KST2>(st + 1, nst, Sk) * kss;
+    const HK_G uint8_t* const vn = Vb + stage_origin<KST2>(st + 1, nst, Sk) * vss;
+    const __amdgpu_buffer_rsrc_t krs = PAD ? edge_rsrc(kn) : dma_rsrc(kn), vrs = PAD ? edge_rsrc(vn) : dma_rsrc(vn);
     const HK_L uint8_t* Kt = BUF ? K1 : K0;
     const HK_L uint8_t* Vt = BUF ? V1 : V0;
     // S^T, dP^T of d step ks; their A operands (K, V rows) are read RA1 steps ahead into a ring, each step
@@ -618,7 +637,7 @@ __global__ __launch_bounds__(512) void attn_dq_dma(hrt_attn_args p, int nqb) {
       acc[i >> 1] = Mfma32<T>::mac(ring[i % (RA + 1)], (i & 1) ? d1 : d0, acc[i >> 1]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
+    barrier_keep_vm_lds<0>();  // waits for this wave's copies, then for every wave
   };
   // Pairs of copying stages, the last one or two peeled into straight-line code (the loop body holds one
   // variant per buffer, which keeps the D = 128 kernel within its 256 registers).
@@ -674,7 +693,7 @@ __global__ __launch_bounds__(512) void attn_dq_dma(hrt_attn_args p, int nqb) {
       const f32x4 v = *reinterpret_cast<const f32x4*>(area + qq * 36 + c4);
       const int64_t qrow = qb * 64 + g * 32 + qq;
       const float v4[4] = {v[0], v[1], v[2], v[3]};
-      if (qrow < Sq)
+      if (qrow < Sq && (!PAD || N * 32 + c4 < p.D))
         *reinterpret_cast<HK_G u32x2*>(gptr<uint16_t>(p.dq) + grad_row(p, b, hh, qrow, Sq, p.q_sb, p.q_sh, p.q_ss) + N * 32 + c4) =
             pack4<T>(v4);
     }
@@ -689,7 +708,7 @@ __global__ __launch_bounds__(512) void attn_dq_dma(hrt_attn_args p, int nqb) {
 
 constexpr int QST = 128;  // queries per LDS stage of the dK / dV kernel
 
-// ---- dK / dV fast path: D = 64 or 128, 16-byte aligned rows -------------------------------------------------
+// ---- dK / dV fast path: D a multiple of 8 above 32, 16-byte aligned rows -------------------------------------------------
 //
 // Per workgroup 64 keys; Q and dO stream through LDS in double-buffered 128-query stages copied global ->
 // LDS directly, with that stage's lse and delta rows beside them.  8 wavefronts on v_mfma_f32_32x32x16:
@@ -710,8 +729,13 @@ constexpr int QST = 128;  // queries per LDS stage of the dK / dV kernel
 // (deterministic), wave (k, q) finishing d block q (D = 128; D = 64: dK blocks by q = 0, 1, dV blocks by
 // q = 2, 3), and store coalesced [key][d] rows.  P and dS are rounded to the input dtype before their
 // products, as attn_coop.comp.in:235-236, 283-284.
-template <typename T, int DCH>
-__global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
+//
+// PAD: as the forward's.  SPLIT: few key blocks (a 77-token context: two per head) would leave most CUs idle, so
+// `splits` workgroups share a key block, each taking a run of query stages and writing fp32 partial dK, dV
+// ([split][b h][key][2][D] in p.o32) that attn_dkdv_sum adds in split order (B2 H8, 1024 queries, 77 keys of 80: 56 us
+// on 32 workgroups of the general kernel; the whole forward + backward 88 -> 47).
+template <typename T, int DCH, bool PAD, bool SPLIT>
+__global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb, int splits) {
   constexpr int NW = 8;
   constexpr int NCH = DCH * 4;        // 16-byte chunks per row
   constexpr int ROWB = NCH * 16;      // bytes per LDS tile row
@@ -734,8 +758,9 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kg = wave & 1, qq = wave >> 1;
   const int rl = lane & 31, hl = lane >> 5;
-  uint32_t bh32, kb32;
-  xcd_map32(blockIdx.x, (uint32_t)nkb * p.B * p.H, nkb, bh32, kb32);
+  uint32_t bh32, kb32, sp = 0;
+  xcd_map32(blockIdx.x, (uint32_t)nkb * p.B * p.H * splits, nkb * splits, bh32, kb32);
+  if constexpr (SPLIT) sp = kb32 / (uint32_t)nkb, kb32 %= (uint32_t)nkb;
   const int64_t bh = bh32, kb = kb32, b = bh32 / (uint32_t)p.H, hh = bh32 % (uint32_t)p.H;
   const int Sq = p.Sq, Sk = p.Sk;
   const uint32_t qss = (uint32_t)(p.q_ss * 2), oss = (uint32_t)(p.do_ss * 2);
@@ -744,6 +769,10 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
   const HK_G float* lseb = gcptr<float>(p.lse) + bh * Sq;
   const HK_G float* dltb = gcptr<float>(p.delta) + bh * Sq;
   const int nst = (Sq + QST - 1) / QST;
+  // this workgroup's stages [st0, st1)
+  const int per = SPLIT ? (nst + splits - 1) / splits : nst, st0 = SPLIT ? (int)sp * per : 0;
+  const int st1 = SPLIT && st0 + per < nst ? st0 + per : nst;
+  const int dch = PAD ? p.D / 8 : NCH;  // chunks of a row that exist
 
   const int j0 = wave * IPW;
   // Values that depend only on the lane are re-derived where they are used from an opaque copy of the lane
@@ -774,13 +803,27 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
                                kb * 64 * (int64_t)kss;
     const HK_G uint8_t* Vblk = reinterpret_cast<const HK_G uint8_t*>(gcptr<uint16_t>(p.v) + b * p.v_sb + hh * p.v_sh) +
                                kb * 64 * (int64_t)vss;
-    dma_tile<NCH, 64, NW>(Kblk, kss, kvalid, Q1, wave, lane, dma_lane_offsets<NCH>(kss, lane, jk));
-    dma_tile<NCH, 64, NW>(Vblk, vss, kvalid, VL, wave, lane, dma_lane_offsets<NCH>(vss, lane, jk));
+    if constexpr (PAD) {
+      edge_tile<NCH, 64, NW>(Kblk, kss, kvalid, dch, Q1, wave, lane);
+      edge_tile<NCH, 64, NW>(Vblk, vss, kvalid, dch, VL, wave, lane);
+    } else {
+      dma_tile<NCH, 64, NW>(Kblk, kss, kvalid, Q1, wave, lane, dma_lane_offsets<NCH>(kss, lane, jk));
+      dma_tile<NCH, 64, NW>(Vblk, vss, kvalid, VL, wave, lane, dma_lane_offsets<NCH>(vss, lane, jk));
+    }
   }
-  issue_order_fence();  // the first barrier counts on stage 0's copies being the last ones issued
-  dma_tile<NCH, QST, NW>(Qb, qss, Sq, Q0, wave, lane, dma_lane_offsets<NCH>(qss, lane, j0));
-  dma_tile<NCH, QST, NW>(Ob, oss, Sq, O0, wave, lane, dma_lane_offsets<NCH>(oss, lane, j0));
-  copy_ls(0, ls_dst(0));
+  issue_order_fence();  // the first barrier counts on the first stage's copies being the last ones issued
+  {
+    const int64_t org = SPLIT && nst > 1 ? stage_origin<QST>(st0, nst, Sq) : 0;
+    const int valid = SPLIT ? (int)(Sq - org) : Sq;
+    if constexpr (PAD) {
+      edge_tile<NCH, QST, NW>(Qb + org * qss, qss, valid, dch, Q0, wave, lane);
+      edge_tile<NCH, QST, NW>(Ob + org * oss, oss, valid, dch, O0, wave, lane);
+    } else {
+      dma_tile<NCH, QST, NW>(Qb + org * qss, qss, valid, Q0, wave, lane, dma_lane_offsets<NCH>(qss, lane, j0));
+      dma_tile<NCH, QST, NW>(Ob + org * oss, oss, valid, O0, wave, lane, dma_lane_offsets<NCH>(oss, lane, j0));
+    }
+  }
+  copy_ls(st0, ls_dst(0));
 
   // per-lane byte offsets inside a 32-row quarter of a tile of the A-operand rows (row rl, chunk 2 ks + h);
   // the tile rows of a quarter start at 32 q, which keeps the swizzle (it uses row bits 0..3)
@@ -804,7 +847,7 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
     HK_L u32x4* v = reinterpret_cast<HK_L u32x4*>(VL) + i;
     *v = *v ^ u32x4{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
   }
-  __syncthreads();  // stage 0 landed; K fragments read and V negated before stage 1 is copied over K
+  barrier_keep_vm_lds<0>();  // the first stage landed; K fragments read and V negated before stage 1 is copied over K
 
   const HK_L uint8_t* const Vq = VL + kg * 32 * ROWB;
   // Stage st from buffer BUF.  Its copies of stage st + 1 are placed between the MFMAs of S / dP (a last
@@ -816,7 +859,7 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
   auto stage = [&](auto bc, auto rc, int st) {
     constexpr int BUF = decltype(bc)::value;
     constexpr bool RAGGED = decltype(rc)::value;
-    const bool COPY = st + 1 < nst;
+    const bool COPY = st + 1 < st1;
     const HK_L uint8_t* Qt = (BUF ? Q1 : Q0) + qq * 32 * ROWB;
     const HK_L uint8_t* Ot = (BUF ? O1 : O0) + qq * 32 * ROWB;
     const float* ls = &ls_raw[BUF][qq * 32 + 4 * hl];
@@ -842,8 +885,9 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
           s[4 * j + r] = qa >= st * QST && qa < Sq ? s[4 * j + r] : -INFINITY;
         }
     }
-    const __amdgpu_buffer_rsrc_t qrs = dma_rsrc(Qb + stage_origin<QST>(st + 1, nst, Sq) * qss);
-    const __amdgpu_buffer_rsrc_t ors = dma_rsrc(Ob + stage_origin<QST>(st + 1, nst, Sq) * oss);
+    const HK_G uint8_t* const qn = Qb + stage_origin<QST>(st + 1, nst, Sq) * qss;
+    const HK_G uint8_t* const on = Ob + stage_origin<QST>(st + 1, nst, Sq) * oss;
+    const __amdgpu_buffer_rsrc_t qrs = PAD ? edge_rsrc(qn) : dma_rsrc(qn), ors = PAD ? edge_rsrc(on) : dma_rsrc(on);
     HK_L uint8_t* const sink = (HK_L uint8_t*)sink_raw;
     HK_L uint8_t* const qdst = COPY ? (BUF ? Q0 : Q1) + j0 * 1024 : sink;
     HK_L uint8_t* const odst = COPY ? (BUF ? O0 : O1) + j0 * 1024 : sink;
@@ -862,8 +906,9 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const uint32_t x = x0 ^ (uint32_t)(tile_swz<NCH>(i * RPI) << 4);
-        qlo.off[i] = bq + x;
-        olo.off[i] = bo + x;
+        const bool in = !PAD || (int)(x >> 4) < dch;
+        qlo.off[i] = in ? bq + x : kNoRow;
+        olo.off[i] = in ? bo + x : kNoRow;
       }
     }
     // S and dP products of d step ks; their operands (Q, dO, V rows) are read RA1 steps ahead into a ring,
@@ -940,12 +985,12 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
         dv[n] = Mfma32<T>::mac(c ? pa1 : pa0, ring[i % (RA + 1)], dv[n]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
+    barrier_keep_vm_lds<0>();  // waits for this wave's copies, then for every wave
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
-  const int nfull = Sq % QST == 0 ? nst : nst - 1;  // stages without ragged rows
-  int st = 0;
+  const int nfull = Sq % QST == 0 || st1 < nst ? st1 : st1 - 1;  // end of the stages without ragged rows
+  int st = st0;
   for (; st + 1 < nfull; st += 2) {
     stage(I0(), std::false_type(), st);
     stage(I1(), std::false_type(), st + 1);
@@ -954,8 +999,8 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
     stage(I0(), std::false_type(), st);
     ++st;
   }
-  if (st < nst) {  // the ragged last stage, in buffer st & 1
-    if (st & 1)
+  if (st < st1) {  // the ragged last stage, in buffer (st - st0) & 1
+    if ((st - st0) & 1)
       stage(I1(), std::true_type(), st);
     else
       stage(I0(), std::true_type(), st);
@@ -1023,6 +1068,15 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
         const f32x4 y = *reinterpret_cast<const f32x4*>(ar + key * 40 + c8 + 4);
         const int64_t kk = kb * 64 + kg * 32 + key;
         const float o8[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+        if (PAD && n * 32 + c8 >= p.D) continue;
+        if constexpr (SPLIT) {
+          HK_G float* const w = gptr<float>(p.o32) + ((((int64_t)sp * p.B * p.H + bh) * Sk + kk) * 2 + R) * p.D + n * 32 + c8;
+          if (kk < Sk) {
+            *reinterpret_cast<HK_G f32x4*>(w) = x;
+            *reinterpret_cast<HK_G f32x4*>(w + 4) = y;
+          }
+          continue;
+        }
         if (kk < Sk)
           *reinterpret_cast<HK_G u32x4*>(gptr<uint16_t>(dst_base) + grad_row(p, b, hh, kk, Sk, g_sb, g_sh, g_ss) + n * 32 + c8) =
               pack8<T>(o8);
@@ -1034,10 +1088,53 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb) {
   round(I1());
 }
 
-// The direct-to-LDS paths need D = 64 or 128, 16-byte aligned rows (q, k, v, dout) and per-stage row
+// dK, dV from the splits' partial products, added in split order: eight d of one (b, h, key) per thread.
+template <typename T>
+__global__ __launch_bounds__(256) void attn_dkdv_sum(hrt_attn_args p, int splits) {
+  const int64_t dc = p.D / 8, rows = (int64_t)p.B * p.H * p.Sk, n = rows * 2 * dc;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int64_t row2 = i / dc, d = (i - row2 * dc) * 8, row = row2 >> 1;
+  const HK_G float* w = gcptr<float>(p.o32) + row2 * p.D + d;
+  f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
+  int s = 0;
+  for (; s + 4 <= splits; s += 4) {  // four splits' loads in flight
+    f32x4 a[4], c[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      a[u] = *reinterpret_cast<const HK_G f32x4*>(w + (s + u) * rows * 2 * p.D);
+      c[u] = *reinterpret_cast<const HK_G f32x4*>(w + (s + u) * rows * 2 * p.D + 4);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x += a[u], y += c[u];
+  }
+  for (; s < splits; ++s) {
+    x += *reinterpret_cast<const HK_G f32x4*>(w + s * rows * 2 * p.D);
+    y += *reinterpret_cast<const HK_G f32x4*>(w + s * rows * 2 * p.D + 4);
+  }
+  const float o8[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+  const int64_t bh = row / p.Sk, key = row - bh * p.Sk, b = bh / p.H, hh = bh - b * p.H;
+  const bool v = row2 & 1;
+  *reinterpret_cast<HK_G u32x4*>(gptr<uint16_t>(v ? p.dv : p.dk) +
+                                 grad_row(p, b, hh, key, p.Sk, v ? p.v_sb : p.k_sb, v ? p.v_sh : p.k_sh, v ? p.v_ss : p.k_ss) + d) = pack8<T>(o8);
+}
+
+// Query splits of the fast dK / dV path: as many as keep its workgroups within one round of 256, whole 128-query stages
+// each.  A split costs its partials' write and read and a launch (~6 us): only where the stages one workgroup
+// would walk take longer (from 3 on, at ~4 us a stage).
+int dkdv_splits(const hrt_attn_args& a) {
+  const int64_t wgs = (int64_t)((a.Sk + 63) / 64) * a.B * a.H, nst = (a.Sq + QST - 1) / QST;
+  if (wgs > 128 || nst < 4) return 1;
+  int64_t s = 256 / wgs;
+  if (s > nst) s = nst;
+  const int64_t per = cdiv(nst, s);
+  return (int)cdiv(nst, per);
+}
+
+// The direct-to-LDS paths need D % 8 == 0 above 32, 16-byte aligned rows (q, k, v, dout) and per-stage row
 // offsets that fit the 32-bit lane offsets of the copies.
 bool bwd_dma_ok(const hrt_attn_args& a) {
-  if (!(a.D == 64 || a.D == 128) || !attn_vec_ok(a, true)) return false;
+  if (a.D <= 32 || !attn_vec_ok(a, true)) return false;
   const int64_t lim = (int64_t)1 << 31;
   return a.k_ss * 2 * (KST2 + 1) < lim && a.v_ss * 2 * (KST2 + 1) < lim && a.q_ss * 2 * (KST2 + 1) < lim &&
          a.do_ss * 2 * (KST2 + 1) < lim;
@@ -1052,11 +1149,22 @@ bool launch_dkdv(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   if (total > 0x7fffffffLL) return ctx.fail("grid too large");
   const dim3 g((uint32_t)total);
   if (bwd_dma_ok(a)) {
-    if (a.D == 128)
-      hipLaunchKernelGGL((attn_dkdv_w32<T, 4>), g, dim3(512), 0, ctx.stream, a, nkb);
-    else
-      hipLaunchKernelGGL((attn_dkdv_w32<T, 2>), g, dim3(512), 0, ctx.stream, a, nkb);
-    return hrt::launch_ok(hipGetLastError(), ctx, "attn_dkdv_w32");
+    const int64_t part = (int64_t)a.B * a.H * a.Sk * 2 * a.D;  // floats of one split's partials
+    const int splits = (a.flags & HRT_ATTN_DKDV_WS) && a.o32 % 16 == 0 ? dkdv_splits(a) : 1;
+    if (splits > 1 && !ctx.check(a.o32, (uint64_t)(part * splits) * 4, "o32")) return false;
+    const dim3 gs((uint32_t)(total * splits));
+#define HK_DKDV(DCH, PAD)                                                                                       \
+  if (splits > 1) hipLaunchKernelGGL((attn_dkdv_w32<T, DCH, PAD, true>), gs, dim3(512), 0, ctx.stream, a, nkb, splits); \
+  else hipLaunchKernelGGL((attn_dkdv_w32<T, DCH, PAD, false>), g, dim3(512), 0, ctx.stream, a, nkb, 1)
+    if (a.D == 128) HK_DKDV(4, false);
+    else if (a.D > 64) HK_DKDV(4, true);
+    else if (a.D == 64) HK_DKDV(2, false);
+    else HK_DKDV(2, true);
+#undef HK_DKDV
+    if (!hrt::launch_ok(hipGetLastError(), ctx, "attn_dkdv_w32")) return false;
+    if (splits > 1)
+      hipLaunchKernelGGL(attn_dkdv_sum<T>, dim3((uint32_t)cdiv(part / 8, 256)), dim3(256), 0, ctx.stream, a, splits);
+    return hrt::launch_ok(hipGetLastError(), ctx, "attn_dkdv_sum");
   }
   const int lm = !attn_vec_ok(a, true) ? LD_GATHER : (a.D % 32 == 0 ? LD_FULL : LD_VEC);
 #define HK_LAUNCH(DCH)                                                                                   \
@@ -1088,17 +1196,21 @@ bool launch_dq(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   const dim3 g((uint32_t)total);
   if (bwd_dma_ok(a)) {
     if (with_delta && !ctx.check(a.o, (uint64_t)a.B * a.H * a.Sq * a.D * (of32 ? 4 : 2), "o")) return false;
-#define HK_DQ(DCH)                                                                                          \
+#define HK_DQ(DCH, PAD)                                                                                     \
   if (!with_delta)                                                                                          \
-    hipLaunchKernelGGL((attn_dq_dma<T, DCH, false, false>), g, dim3(512), 0, ctx.stream, a, nqb);            \
+    hipLaunchKernelGGL((attn_dq_dma<T, DCH, false, false, PAD>), g, dim3(512), 0, ctx.stream, a, nqb);       \
   else if (of32)                                                                                            \
-    hipLaunchKernelGGL((attn_dq_dma<T, DCH, true, true>), g, dim3(512), 0, ctx.stream, a, nqb);              \
+    hipLaunchKernelGGL((attn_dq_dma<T, DCH, true, true, PAD>), g, dim3(512), 0, ctx.stream, a, nqb);         \
   else                                                                                                      \
-    hipLaunchKernelGGL((attn_dq_dma<T, DCH, false, true>), g, dim3(512), 0, ctx.stream, a, nqb);
+    hipLaunchKernelGGL((attn_dq_dma<T, DCH, false, true, PAD>), g, dim3(512), 0, ctx.stream, a, nqb);
     if (a.D == 128) {
-      HK_DQ(4)
+      HK_DQ(4, false)
+    } else if (a.D > 64) {
+      HK_DQ(4, true)
+    } else if (a.D == 64) {
+      HK_DQ(2, false)
     } else {
-      HK_DQ(2)
+      HK_DQ(2, true)
     }
 #undef HK_DQ
     return hrt::launch_ok(hipGetLastError(), ctx, "attn_dq_dma");
@@ -1129,3 +1241,9 @@ HRT_REGISTER("attn_dq_mfma_f16", hrt_attn_args, launch_dq<F16>);
 
 }  // namespace
 }  // namespace hk
+
+extern "C" int64_t hrt_attn_dkdv_workspace(const hrt_attn_args* a) {
+  if (a == nullptr || a->B < 1 || a->H < 1 || a->Sq < 1 || a->Sk < 1 || !hk::bwd_dma_ok(*a)) return 0;
+  const int s = hk::dkdv_splits(*a);
+  return s > 1 ? (int64_t)s * a->B * a->H * a->Sk * 2 * a->D : 0;
+}

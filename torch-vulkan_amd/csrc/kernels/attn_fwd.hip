@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(hrt_attn_args p, int nqb) {
     }
 }
 
-// ---- fast path: D = 64 or 128, 16-byte aligned rows ---------------------------------------------------------
+// ---- fast path: D a multiple of 8 above 32, 16-byte aligned rows ---------------------------------------------------------
 //
 // Differences from the general kernel above:
 //   * K and V stages go global -> LDS directly (global_load_lds_dwordx4): no staging registers and no
@@ -231,7 +231,9 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(hrt_attn_args p, int nqb) {
 //     d block k of group g.
 constexpr float kLazy = 8.f;  // log2 of the largest unnormalised P value
 
-template <typename T, int DCH>
+// PAD: D is a multiple of 8 below the tile width 32 DCH; the missing columns are zeros in LDS (masked copy lanes) and
+// are not stored.
+template <typename T, int DCH, bool PAD>
 __global__ __launch_bounds__(512) void attn_fwd_dma(hrt_attn_args p, int nqb) {
   constexpr int NW = 8;               // wavefronts
   constexpr int NCH = DCH * 4;        // 16-byte chunks per row
@@ -262,7 +264,9 @@ __global__ __launch_bounds__(512) void attn_fwd_dma(hrt_attn_args p, int nqb) {
   const int nst = (Sk + KST - 1) / KST;
 
   const int j0 = wave * (KST * NCH / 64 / NW);
-  const DmaLanes klo = dma_lane_offsets<NCH>(kss, lane, j0), vlo = dma_lane_offsets<NCH>(vss, lane, j0);
+  const int dch = PAD ? p.D / 8 : NCH;  // chunks of a row that exist
+  const DmaLanes klo = PAD ? edge_lanes<NCH>(kss, lane, j0, dch) : dma_lane_offsets<NCH>(kss, lane, j0);
+  const DmaLanes vlo = PAD ? edge_lanes<NCH>(vss, lane, j0, dch) : dma_lane_offsets<NCH>(vss, lane, j0);
   // The block's 64 Q rows go to V(1)'s buffer (free until stage 0 copies V(1)), copied once for the four
   // wavefronts that share them; then K(0), V(0) and K(1): K streams one stage ahead of V
   const uint32_t qss = (uint32_t)(p.q_ss * 2);
@@ -270,12 +274,21 @@ __global__ __launch_bounds__(512) void attn_fwd_dma(hrt_attn_args p, int nqb) {
                              qb * 64 * (int64_t)qss;
   const int64_t q = qb * 64 + g * 32 + ql;
   u32x4 qf[2 * DCH];  // Q^T operand fragments of this lane's query, read from LDS after the first barrier
-  dma_tile<NCH, 64, NW>(Qblk, qss, (int)(Sq - qb * 64), V1, wave, lane,
-                        dma_lane_offsets<NCH>(qss, lane, wave * (64 * NCH / 64 / NW)));
-  dma_tile<NCH, KST, NW>(Kb, kss, Sk, K0, wave, lane, klo);
-  dma_tile<NCH, KST, NW>(Vb, vss, Sk, V0, wave, lane, vlo);
+  if constexpr (PAD) {
+    edge_tile<NCH, 64, NW>(Qblk, qss, (int)(Sq - qb * 64), dch, V1, wave, lane);
+    edge_tile<NCH, KST, NW>(Kb, kss, Sk, dch, K0, wave, lane);
+    edge_tile<NCH, KST, NW>(Vb, vss, Sk, dch, V0, wave, lane);
+  } else {
+    dma_tile<NCH, 64, NW>(Qblk, qss, (int)(Sq - qb * 64), V1, wave, lane,
+                          dma_lane_offsets<NCH>(qss, lane, wave * (64 * NCH / 64 / NW)));
+    dma_tile<NCH, KST, NW>(Kb, kss, Sk, K0, wave, lane, klo);
+    dma_tile<NCH, KST, NW>(Vb, vss, Sk, V0, wave, lane, vlo);
+  }
   issue_order_fence();  // the first barrier counts on K(1) being the last copy issued
-  if (nst > 1) dma_tile<NCH, KST, NW>(Kb + stage_origin<KST>(1, nst, Sk) * kss, kss, KST, K1, wave, lane, klo);
+  if (nst > 1) {
+    if constexpr (PAD) edge_tile<NCH, KST, NW>(Kb + stage_origin<KST>(1, nst, Sk) * kss, kss, KST, dch, K1, wave, lane);
+    else dma_tile<NCH, KST, NW>(Kb + stage_origin<KST>(1, nst, Sk) * kss, kss, KST, K1, wave, lane, klo);
+  }
 
   // per-lane byte offsets of the A-operand fragments inside a tile
   int koff[2 * DCH], voff[DCH][2];
@@ -355,8 +368,10 @@ __global__ __launch_bounds__(512) void attn_fwd_dma(hrt_attn_args p, int nqb) {
     if constexpr (COPY) {
       // buffer resources over the stages' first rows: a copy then takes its row offset in a scalar register
       // and its lane offset as is, with no per-copy 64-bit address arithmetic
-      const __amdgpu_buffer_rsrc_t krs = dma_rsrc(Kb + stage_origin<KST>(st + 2, nst, Sk) * kss);
-      const __amdgpu_buffer_rsrc_t vrs = dma_rsrc(Vb + stage_origin<KST>(st + 1, nst, Sk) * vss);
+      const HK_G uint8_t* const kn = Kb + stage_origin<KST>(st + 2, nst, Sk) * kss;
+      const HK_G uint8_t* const vn = Vb + stage_origin<KST>(st + 1, nst, Sk) * vss;
+      const __amdgpu_buffer_rsrc_t krs = PAD ? edge_rsrc(kn) : dma_rsrc(kn);
+      const __amdgpu_buffer_rsrc_t vrs = PAD ? edge_rsrc(vn) : dma_rsrc(vn);
       // S(st+1) with this iteration's copies placed after its MFMAs, one per MFMA, then P(st); the VALU
       // work of P(st) is interleaved with the MFMAs by sched_group_barrier
       const HK_L uint8_t* Kt = BUF ? K0 : K1;
@@ -402,11 +417,11 @@ __global__ __launch_bounds__(512) void attn_fwd_dma(hrt_attn_args p, int nqb) {
         o[n] = Mfma32<T>::mac(u32x4{lo.x, lo.y, hi.x, hi.y}, kc ? pb1 : pb0, o[n]);
       }
     if (COPY && st + 1 < nst) mask_and_max(sn, st + 1);
-    __syncthreads();  // waits for this wave's copies, then for every wave
+    barrier_keep_vm_lds<0>();  // waits for this wave's copies, then for every wave
   };
   // Q, K(0), V(0) landed (K(1), issued last, may still be in flight)
   if (nst > 1) barrier_keep_vm<KST * NCH / 64 / NW>();
-  else __syncthreads();
+  else barrier_keep_vm_lds<0>();
   // (rows past Sq hold copies of the last row; their results are never stored)
 #pragma unroll
   for (int ks = 0; ks < 2 * DCH; ++ks)
@@ -503,7 +518,7 @@ __global__ __launch_bounds__(512) void attn_fwd_dma(hrt_attn_args p, int nqb) {
       const int qq = ps * 8 + (lane >> 3);
       const f32x4 v = *reinterpret_cast<const f32x4*>(area + qq * 36 + c4);
       const int64_t qrow = qb * 64 + g * 32 + qq;
-      if (qrow < Sq) {
+      if (qrow < Sq && (!PAD || N * 32 + c4 < p.D)) {
         const int64_t off = ((b * Sq + qrow) * p.H + hh) * p.D + N * 32 + c4;
         const float v4[4] = {v[0], v[1], v[2], v[3]};
         *reinterpret_cast<HK_G u32x2*>(gptr<typename T::storage>(p.o) + off) = pack4<T>(v4);
@@ -519,10 +534,10 @@ __global__ __launch_bounds__(512) void attn_fwd_dma(hrt_attn_args p, int nqb) {
   }
 }
 
-// The direct-to-LDS path needs D = 64 or 128, 16-byte aligned rows, and per-stage row offsets that fit
+// The direct-to-LDS path needs 16-byte aligned rows of whole 16-byte chunks (D % 8 == 0) and more than 32 columns, and per-stage row offsets that fit
 // the 32-bit lane offsets of the copies.
 bool fwd_dma_ok(const hrt_attn_args& a) {
-  if (!(a.D == 64 || a.D == 128) || !attn_vec_ok(a, false)) return false;
+  if (a.D <= 32 || !attn_vec_ok(a, false)) return false;
   const int64_t lim = (int64_t)1 << 31;
   return a.k_ss * 2 * (KST + 1) < lim && a.v_ss * 2 * (KST + 1) < lim && a.q_ss * 2 * (64 + 1) < lim;
 }
@@ -536,10 +551,12 @@ bool launch_fwd(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   if (total > 0x7fffffffLL) return ctx.fail("grid too large");
   const dim3 g((uint32_t)total);
   if (fwd_dma_ok(a)) {
-    if (a.D == 128)
-      hipLaunchKernelGGL((attn_fwd_dma<T, 4>), g, dim3(512), 0, ctx.stream, a, nqb);
-    else
-      hipLaunchKernelGGL((attn_fwd_dma<T, 2>), g, dim3(512), 0, ctx.stream, a, nqb);
+    // 65 to 96 columns pay for 128: the 96-wide rows of the general kernel's tiles have no copy swizzle, and it is
+    // slower all the same (forward + backward at B1 H4 S1395 D80: 170 us there, 59 on padded tiles)
+    if (a.D == 128) hipLaunchKernelGGL((attn_fwd_dma<T, 4, false>), g, dim3(512), 0, ctx.stream, a, nqb);
+    else if (a.D > 64) hipLaunchKernelGGL((attn_fwd_dma<T, 4, true>), g, dim3(512), 0, ctx.stream, a, nqb);
+    else if (a.D == 64) hipLaunchKernelGGL((attn_fwd_dma<T, 2, false>), g, dim3(512), 0, ctx.stream, a, nqb);
+    else hipLaunchKernelGGL((attn_fwd_dma<T, 2, true>), g, dim3(512), 0, ctx.stream, a, nqb);
     return hrt::launch_ok(hipGetLastError(), ctx, "attn_fwd_dma");
   }
   const int lm = !attn_vec_ok(a, false) ? LD_GATHER : (a.D % 32 == 0 ? LD_FULL : LD_VEC);

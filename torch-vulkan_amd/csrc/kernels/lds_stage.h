@@ -195,6 +195,28 @@ __device__ __forceinline__ void edge_copy(__amdgpu_buffer_rsrc_t rs, HK_L uint8_
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, tile + j * 1024, 16, (int)off, 0, 0, 0);
 }
 
+// A ROWS x NCH-chunk tile whose rows hold only c_hi chunks (the rest reads zeros) and whose rows [valid, ROWS) are zeros,
+// copied by NW wavefronts.
+template <int NCH, int ROWS, int NW>
+__device__ __forceinline__ void edge_tile(const HK_G uint8_t* src, uint32_t ss, int valid, int c_hi, HK_L uint8_t* tile, int wave,
+                                          int lane) {
+  constexpr int IPW = ROWS * NCH / 64 / NW;
+  uint32_t off[IPW];
+  edge_lane_offsets<NCH, IPW>(off, ss, lane, wave * IPW, 0, valid < ROWS ? valid : ROWS, 0, c_hi);
+  const __amdgpu_buffer_rsrc_t rs = edge_rsrc(src);
+#pragma unroll
+  for (int i = 0; i < IPW; ++i) edge_copy(rs, tile, wave * IPW + i, off[i]);
+}
+// dma_lane_offsets with the lanes of chunks c_hi and up masked, for dma_tile_part_rs on an edge_rsrc resource.
+template <int NCH>
+__device__ __forceinline__ DmaLanes edge_lanes(uint32_t ss, int lane, int j0, int c_hi) {
+  DmaLanes d = dma_lane_offsets<NCH>(ss, lane, j0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (((lane % NCH) ^ tile_swz<NCH>((j0 + i) * (64 / NCH) + lane / NCH)) >= c_hi) d.off[i] = kNoRow;
+  return d;
+}
+
 // First row of the tile that stage st copies when the sequence has more than one stage (len > ROWS): stage
 // st covers rows [st ROWS, (st + 1) ROWS); the last, ragged stage copies the full window that ends at row
 // len - 1 instead (origin len - ROWS), so no copy reads past the sequence, and its rows below st ROWS

@@ -218,6 +218,12 @@ BwdOut k_sdpa_bwd(const at::Tensor& grad_out, const at::Tensor& query, const at:
     hrt_attn_args KV = A;
     KV.dk = dptr(dk);
     KV.dv = dptr(dv);
+    at::Tensor partial;  // few key blocks: partial dK, dV of query ranges
+    if (const int64_t ws = matrix_cores(dt) ? hrt_attn_dkdv_workspace(&KV) : 0; ws > 0) {
+      partial = at::empty({ws}, q.options().dtype(at::kFloat));
+      KV.o32 = dptr(partial);
+      KV.flags |= HRT_ATTN_DKDV_WS;
+    }
     queue(attn_kernel("dkdv", dt), KV);
     note_gpu(kBwdOp);
   }
