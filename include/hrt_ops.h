@@ -382,6 +382,24 @@ static inline int64_t hrt_conv3_splits(int64_t N, int64_t I, int64_t O, int64_t 
   while (tiles * s * 2 <= 256 && nb % (2 * s) == 0 && nb / (2 * s) >= 4) s *= 2;
   return s;
 }
+/* "conv3x3r_wprep_{bf16,f16}" and "conv3x3r_{bf16,f16}" — the same convolution for O a multiple of 32 and W of 8: four
+ * output rows x 32 pixels per workgroup, the last block of output channels padded to 128 by zero rows of wr, which
+ * holds hrt_conv3r_wr_bytes(O, I) bytes. */
+static inline int64_t hrt_conv3r_wr_bytes(int64_t O, int64_t I) { return hrt_conv3_wr_bytes((O + 127) / 128 * 128, I); }
+/* Input-channel split of "conv3x3r_{dt}": the cheapest of the divisors of I / 16 that leave 4 channel blocks, a round
+ * of 256 workgroups taking ~1.6 us a block and a split its partial sums' write and read and a launch. */
+static inline int64_t hrt_conv3r_splits(int64_t N, int64_t I, int64_t O, int64_t H, int64_t W) {
+  const int64_t tiles = N * ((H + 3) / 4) * ((W + 31) / 32) * ((O + 127) / 128), nb = I / 16;
+  int64_t best = 1;
+  double best_us = 0.0;
+  for (int64_t s = 1; s <= 8 && (s == 1 || nb / s >= 4); ++s) {
+    if (nb % s != 0) continue;
+    double us = (double)((tiles * s + 255) / 256) * (double)(nb / s) * 1.6;
+    if (s > 1) us += 3.0 + 1.3e-6 * (double)(s * N * O) * (double)(H * W);
+    if (s == 1 || us < best_us) best_us = us, best = s;
+  }
+  return best;
+}
 typedef struct hrt_conv3_wprep_args {
   uint64_t w, wr;
   int64_t O, I;

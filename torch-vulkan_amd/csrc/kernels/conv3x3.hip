@@ -52,6 +52,14 @@ __global__ __launch_bounds__(256) void conv3_wprep_k(hrt_conv3_wprep_args a) {
   const int tid = threadIdx.x;
   const int64_t nb = a.I / C3_CB, o0 = (int64_t)blockIdx.x * 32, cb = blockIdx.y;
   const HK_G uint16_t* w = gcptr<uint16_t>(a.w);
+  if (o0 >= a.O) {  // the padding rows of the last block (ragged O)
+    for (int k = tid; k < 32 * 19; k += 256) {
+      const int64_t og = o0 + k / 19;
+      HK_G uint16_t* row = gptr<uint16_t>(a.wr) + (((og / C3_CO) * nb + cb) * C3_CO + og % C3_CO) * C3_ARS;
+      *reinterpret_cast<HK_G u32x4*>(row + (k % 19) * 8) = u32x4{0, 0, 0, 0};
+    }
+    return;
+  }
   u32x4 v[3];
 #pragma unroll
   for (int j = 0; j < 3; ++j) {  // pieces k = tid + 256 j < 576, all loads issued before the stores
@@ -230,8 +238,150 @@ __global__ __launch_bounds__(512) void conv3_igemm_k(hrt_conv3_args p) {
   }
 }
 
+// Ragged form (any O % 32 == 0 with the weight tiles of the last block padded by zeros, any W % 8 == 0): a workgroup
+// owns 128 output channels x four output rows x a 32-pixel segment, so a 96-pixel row is three whole segments, and a
+// wavefront's two accumulators are two rows, whose three taps along H share staged rows: 9 + 12 fragment reads per
+// step for 18 MFMAs against 9 + 18 in the 64-pixel form.
+constexpr int C3R_PX = 32, C3R_ROWS = 4, C3R_SROWS = C3R_ROWS + 2, C3R_BCOLS = C3R_PX + 2;
+constexpr int C3R_BTILE = C3R_SROWS * C3R_BCOLS * C3_BPS;
+template <typename T>
+__global__ __launch_bounds__(512) void conv3_ragged_k(hrt_conv3_args p) {
+  __shared__ __attribute__((aligned(16))) uint8_t a0_raw[C3_ASLAB], a1_raw[C3_ASLAB];
+  __shared__ __attribute__((aligned(16))) uint16_t b0_raw[C3R_BTILE], b1_raw[C3R_BTILE];
+  HK_L uint8_t* const A0 = (HK_L uint8_t*)a0_raw;
+  HK_L uint8_t* const A1 = (HK_L uint8_t*)a1_raw;
+  HK_L uint16_t* const B0 = (HK_L uint16_t*)b0_raw;
+  HK_L uint16_t* const B1 = (HK_L uint16_t*)b1_raw;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave & 3, wr = wave >> 2, l32 = lane & 31, hh = lane >> 5;
+  const int64_t H = p.H, W = p.W, I = p.I, O = p.O;
+  const int64_t nb = I / C3_CB, S = p.splits, steps = nb / S;
+  const int64_t segs = cdiv(W, C3R_PX), rquads = cdiv(H, C3R_ROWS), ncob = cdiv(O, C3_CO), combos = ncob * S;
+  const uint32_t bid = blockIdx.x;
+  const uint32_t combo = bid % (uint32_t)combos, unit = bid / (uint32_t)combos;
+  const int64_t cob = combo % ncob, sp = combo / ncob;
+  const int64_t n = unit / (segs * rquads), rs = unit - n * segs * rquads;
+  const int64_t h0 = (rs / segs) * C3R_ROWS, w0 = (rs - (rs / segs) * segs) * C3R_PX;
+  const int64_t co0 = cob * C3_CO, cb0 = sp * steps;
+  const int64_t cstride = (int64_t)C3_CB * H * W;
+  const HK_G uint16_t* X = gcptr<uint16_t>(p.x) + n * I * H * W + cb0 * cstride;
+  const HK_G uint8_t* WR = gcptr<uint8_t>(p.wr) + (cob * nb + cb0) * (int64_t)C3_ASLAB;
+
+  // as conv3_igemm_k: weight pieces tid + 512 k; vector bv (8 pixels, whole inside or outside the row: W % 8 == 0) of
+  // input row h0 - 1 + brow of channel bi (wavefronts 0..5); halo pixel hside of row hrow of channel hi (0..2)
+  const int bi = lane & 15, bv = 2 * (wave & 1) + ((lane >> 4) & 1), brow = 2 * (wave >> 1) + ((lane >> 5) & 1);
+  const int hi = lane & 15, hside = (lane >> 4) & 1, hrow = 2 * wave + ((lane >> 5) & 1);
+  const int64_t bh = h0 - 1 + brow, hr2 = h0 - 1 + hrow, hw = hside ? w0 + C3R_PX : w0 - 1;
+  const bool b_mine = wave < 6, h_mine = wave < 3;
+  const bool b_ok = b_mine && bh >= 0 && bh < H && w0 + bv * 8 < W;
+  const bool h_ok = h_mine && hr2 >= 0 && hr2 < H && hw >= 0 && hw < W;
+  const int64_t boff = b_ok ? (bi * H + bh) * W + w0 + bv * 8 : 0;
+  const int64_t hoff = h_ok ? (hi * H + hr2) * W + hw : 0;
+  const int bdst = (brow * C3R_BCOLS + 1 + bv * 8) * C3_BPS + bi;
+  const int hdst = (hrow * C3R_BCOLS + (hside ? C3R_BCOLS - 1 : 0)) * C3_BPS + hi;
+
+  struct Regs {
+    u32x4 a[C3_AREGS];
+    u32x4 b;
+    uint32_t h;
+  };
+  auto load = [&](int64_t j, Regs& r) {
+    const HK_G uint8_t* wt = WR + j * (int64_t)C3_ASLAB;
+#pragma unroll
+    for (int k = 0; k < C3_AREGS; ++k) {
+      const int pc = tid + 512 * k < C3_APIECES ? tid + 512 * k : C3_APIECES - 1;
+      r.a[k] = *reinterpret_cast<const HK_G u32x4*>(wt + pc * 16);
+    }
+    const HK_G uint16_t* xb = X + j * cstride;
+    r.b = *reinterpret_cast<const HK_G u32x4*>(xb + boff);
+    r.h = xb[hoff];
+  };
+  auto store = [&](HK_L uint8_t* At, HK_L uint16_t* Bt, const Regs& r) {
+#pragma unroll
+    for (int k = 0; k < C3_AREGS; ++k)
+      if (tid + 512 * k < C3_APIECES) *reinterpret_cast<HK_L u32x4*>(At + (tid + 512 * k) * 16) = r.a[k];
+    if (b_mine) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t v = b_ok ? r.b[j] : 0u;
+        Bt[bdst + (2 * j) * C3_BPS] = (uint16_t)(v & 0xffffu);
+        Bt[bdst + (2 * j + 1) * C3_BPS] = (uint16_t)(v >> 16);
+      }
+    }
+    if (h_mine) Bt[hdst] = (uint16_t)(h_ok ? r.h : 0u);
+  };
+
+  f32x16 acc[2] = {zero16(), zero16()};  // output rows h0 + 2 wr, + 1
+  const int aoff = (wm * 32 + l32) * (C3_ARS * 2) + 16 * hh;                 // bytes
+  const int boff_f = (2 * wr * C3R_BCOLS + l32) * C3_BPS + 8 * hh;          // elements
+  Regs r0, r1;
+  auto step = [&](auto sc, int64_t i) {
+    constexpr int SB = decltype(sc)::value;
+    load(i + 2 < steps ? i + 2 : steps - 1, SB == 0 ? r0 : r1);
+    issue_order_fence();  // keeps the loads here, in flight during the MFMAs
+    const HK_L uint8_t* At = SB == 0 ? A0 : A1;
+    const HK_L uint16_t* Bt = SB == 0 ? B0 : B1;
+#pragma unroll
+    for (int kw = 0; kw < 3; ++kw) {
+      u32x4 b[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) b[r] = *reinterpret_cast<const HK_L u32x4*>(Bt + boff_f + (r * C3R_BCOLS + kw) * C3_BPS);
+#pragma unroll
+      for (int kh = 0; kh < 3; ++kh) {
+        const u32x4 a = *reinterpret_cast<const HK_L u32x4*>(At + aoff + (3 * kh + kw) * 32);
+        acc[0] = Mfma32<T>::mac(a, b[kh], acc[0]);
+        acc[1] = Mfma32<T>::mac(a, b[kh + 1], acc[1]);
+      }
+    }
+    if (i + 1 < steps) {
+      if constexpr (SB == 0) store(A1, B1, r1);
+      else store(A0, B0, r0);
+    }
+    barrier_keep_vm_lds<C3_AREGS + 2>();
+  };
+  load(0, r0);
+  load(steps > 1 ? 1 : 0, r1);
+  store(A0, B0, r0);
+  barrier_keep_vm_lds<C3_AREGS + 2>();
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  int64_t i = 0;
+  for (; i + 2 <= steps; i += 2) {
+    step(I0(), i);
+    step(I1(), i + 1);
+  }
+  if (i < steps) step(I0(), i);
+
+  // lane holds out[co0 + wm 32 + 8 j + 4 hh + r][row h0 + 2 wr + u][pixel w0 + l32] in element 4 j + r of acc[u]
+  if (co0 + wm * 32 >= O || w0 + l32 >= W) return;
+  const int64_t HW = H * W;
+  float bv2[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) bv2[e] = 0.f;
+  if (S == 1 && p.has_bias) {  // all 16 loads issued before the first use
+    const HK_G uint16_t* bias = gcptr<uint16_t>(p.bias) + co0 + wm * 32 + 4 * hh;
+    uint16_t braw[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) braw[e] = bias[8 * (e >> 2) + (e & 3)];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) bv2[e] = T::to_f32(braw[e]);
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int64_t row = h0 + 2 * wr + u;
+    if (row >= H) continue;
+    const int64_t px = row * W + w0 + l32;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int64_t co = co0 + wm * 32 + 8 * (e >> 2) + 4 * hh + (e & 3);
+      if (S == 1) gptr<uint16_t>(p.y)[(n * O + co) * HW + px] = T::from_f32(acc[u][e] + bv2[e]);
+      else gptr<float>(p.ws)[((sp * p.N + n) * O + co) * HW + px] = acc[u][e];
+    }
+  }
+}
+
 // y = round(sum over splits s, in order, of ws[s] + bias): 8 consecutive outputs per thread (H W is a
-// multiple of 64, so they share an output channel), 16-byte loads and store.
+// multiple of 8, so they share an output channel), 16-byte loads and store.
 template <typename T>
 __global__ __launch_bounds__(256) void conv3_reduce_k(hrt_conv3_args p) {
   const int64_t HW = p.H * p.W, total = p.N * p.O * HW;
@@ -255,41 +405,52 @@ __global__ __launch_bounds__(256) void conv3_reduce_k(hrt_conv3_args p) {
   *reinterpret_cast<HK_G u32x4*>(gptr<uint16_t>(p.y) + i0) = o;
 }
 
+// RAGGED: O any multiple of 32, padded to whole blocks of 128.
+template <bool RAGGED>
 bool conv3_wprep_launch(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   const auto& a = *static_cast<const hrt_conv3_wprep_args*>(pp);
-  if (a.O <= 0 || a.I <= 0 || a.I % C3_CB != 0 || a.O % C3_CO != 0)
-    return ctx.fail("O must be a positive multiple of 128 and I of 16");
+  if (a.O <= 0 || a.I <= 0 || a.I % C3_CB != 0 || a.O % (RAGGED ? 32 : C3_CO) != 0)
+    return ctx.fail(RAGGED ? "O must be a positive multiple of 32 and I of 16" : "O must be a positive multiple of 128 and I of 16");
+  const int64_t Op = cdiv(a.O, C3_CO) * C3_CO;
   if (a.flip > 1) return ctx.fail("flip must be 0 or 1");
   if (a.w % 16 != 0 || a.wr % 16 != 0) return ctx.fail("w and wr must be 16-byte aligned");
   if (a.O / 32 > 0x7fffffffLL || a.I / C3_CB > 65535) return ctx.fail("grid too large");
-  if (!ctx.check(a.w, (uint64_t)a.O * a.I * 9 * 2, "w") || !ctx.check(a.wr, (uint64_t)hrt_conv3_wr_bytes(a.O, a.I), "wr"))
+  if (!ctx.check(a.w, (uint64_t)a.O * a.I * 9 * 2, "w") || !ctx.check(a.wr, (uint64_t)hrt_conv3_wr_bytes(Op, a.I), "wr"))
     return false;
-  hipLaunchKernelGGL(conv3_wprep_k, dim3((uint32_t)(a.O / 32), (uint32_t)(a.I / C3_CB)), dim3(256), 0, ctx.stream, a);
+  hipLaunchKernelGGL(conv3_wprep_k, dim3((uint32_t)(Op / 32), (uint32_t)(a.I / C3_CB)), dim3(256), 0, ctx.stream, a);
   return hrt::launch_ok(hipGetLastError(), ctx, "conv3x3_wprep");
 }
 
+template <bool RAGGED>
+int64_t conv3_grid(const hrt_conv3_args& a) {
+  const int64_t units = RAGGED ? a.N * cdiv(a.H, C3R_ROWS) * cdiv(a.W, C3R_PX) : a.N * ((a.H + 1) / 2) * (a.W / C3_PX);
+  return units * cdiv(a.O, C3_CO) * a.splits;
+}
+
+template <bool RAGGED>
 bool conv3_check(const hrt_conv3_args& a, hrt::LaunchCtx& ctx) {
   if (a.N <= 0 || a.H <= 0 || a.W <= 0 || a.I <= 0 || a.O <= 0) return ctx.fail("sizes must be positive");
-  if (a.I % C3_CB || a.O % C3_CO || a.W % C3_PX)
-    return ctx.fail("I must be a multiple of 16, O of 128 and W of 64");
+  if (a.I % C3_CB || a.O % (RAGGED ? 32 : C3_CO) || a.W % (RAGGED ? 8 : C3_PX))
+    return ctx.fail(RAGGED ? "I must be a multiple of 16, O of 32 and W of 8" : "I must be a multiple of 16, O of 128 and W of 64");
   if (a.splits < 1 || (a.I / C3_CB) % a.splits) return ctx.fail("splits must divide I / 16");
   if (a.x % 16 || a.wr % 16 || a.y % 16 || (a.has_bias && a.bias % 2) || (a.splits > 1 && a.ws % 16))
     return ctx.fail("misaligned operand");
-  const int64_t units = a.N * ((a.H + 1) / 2) * (a.W / C3_PX), combos = (a.O / C3_CO) * a.splits;
-  if (units * combos > 0x7fffffffLL) return ctx.fail("grid too large");
+  const int64_t Op = cdiv(a.O, C3_CO) * C3_CO;
+  if (conv3_grid<RAGGED>(a) > 0x7fffffffLL) return ctx.fail("grid too large");
   const uint64_t xb = (uint64_t)a.N * a.I * a.H * a.W * 2, yb = (uint64_t)a.N * a.O * a.H * a.W * 2;
-  return ctx.check(a.x, xb, "x") && ctx.check(a.y, yb, "y") && ctx.check(a.wr, (uint64_t)hrt_conv3_wr_bytes(a.O, a.I), "wr") &&
+  return ctx.check(a.x, xb, "x") && ctx.check(a.y, yb, "y") && ctx.check(a.wr, (uint64_t)hrt_conv3_wr_bytes(Op, a.I), "wr") &&
          (!a.has_bias || ctx.check(a.bias, (uint64_t)a.O * 2, "bias")) &&
          (a.splits == 1 || ctx.check(a.ws, yb * 2 * a.splits, "ws"));
 }
 
 // The convolution, and with splits > 1 the reduction of its partial sums right behind it.
-template <typename T>
+template <typename T, bool RAGGED>
 bool conv3_launch(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   const auto& a = *static_cast<const hrt_conv3_args*>(pp);
-  if (!conv3_check(a, ctx)) return false;
-  const int64_t units = a.N * ((a.H + 1) / 2) * (a.W / C3_PX), combos = (a.O / C3_CO) * a.splits;
-  hipLaunchKernelGGL(conv3_igemm_k<T>, dim3((uint32_t)(units * combos)), dim3(512), 0, ctx.stream, a);
+  if (!conv3_check<RAGGED>(a, ctx)) return false;
+  const dim3 g((uint32_t)conv3_grid<RAGGED>(a));
+  if constexpr (RAGGED) hipLaunchKernelGGL(conv3_ragged_k<T>, g, dim3(512), 0, ctx.stream, a);
+  else hipLaunchKernelGGL(conv3_igemm_k<T>, g, dim3(512), 0, ctx.stream, a);
   if (!hrt::launch_ok(hipGetLastError(), ctx, "conv3x3")) return false;
   if (a.splits == 1) return true;
   const int64_t total = a.N * a.O * a.H * a.W;
@@ -297,10 +458,15 @@ bool conv3_launch(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   return hrt::launch_ok(hipGetLastError(), ctx, "conv3x3_reduce");
 }
 
-HRT_REGISTER("conv3x3_wprep_bf16", hrt_conv3_wprep_args, conv3_wprep_launch);
-HRT_REGISTER("conv3x3_wprep_f16", hrt_conv3_wprep_args, conv3_wprep_launch);
-HRT_REGISTER("conv3x3_bf16", hrt_conv3_args, conv3_launch<BF16>);
-HRT_REGISTER("conv3x3_f16", hrt_conv3_args, conv3_launch<F16>);
+HRT_REGISTER("conv3x3_wprep_bf16", hrt_conv3_wprep_args, conv3_wprep_launch<false>);
+HRT_REGISTER("conv3x3_wprep_f16", hrt_conv3_wprep_args, conv3_wprep_launch<false>);
+HRT_REGISTER("conv3x3_bf16", hrt_conv3_args, (conv3_launch<BF16, false>));
+HRT_REGISTER("conv3x3_f16", hrt_conv3_args, (conv3_launch<F16, false>));
+
+HRT_REGISTER("conv3x3r_wprep_bf16", hrt_conv3_wprep_args, conv3_wprep_launch<true>);
+HRT_REGISTER("conv3x3r_wprep_f16", hrt_conv3_wprep_args, conv3_wprep_launch<true>);
+HRT_REGISTER("conv3x3r_bf16", hrt_conv3_args, (conv3_launch<BF16, true>));
+HRT_REGISTER("conv3x3r_f16", hrt_conv3_args, (conv3_launch<F16, true>));
 
 }  // namespace
 }  // namespace hk

@@ -89,38 +89,62 @@ at::Tensor cols_of(const at::Tensor& input, const ConvShape& g) {
 // / writes (swapped for the adjoint).  x, w: the operands the kernel would read, which it takes at 16-byte
 // aligned addresses only (a view at an odd offset, e.g. a weight inside a flat parameter buffer, goes to the
 // unfolding + GEMM path, which takes any alignment).
-bool conv3_ok(const ConvShape& g, at::ScalarType t, int64_t in_ch, int64_t out_ch, const at::Tensor& x, const at::Tensor& w) {
+// Which form of the direct kernel: kExact above; kRagged ("conv3x3r_{dt}") for output channels in multiples of 32 from
+// 128 and rows of a multiple of 8 pixels, where an estimate of its time (rounds of 256 workgroups, ~1.6 us a channel
+// block, padding included) is 5% below that of the unfolding (the column matrix at 2.8 TB/s, its adjoint at 2.2, the
+// product at 600 TFLOP/s).  Measured, direct against unfolded, forward / input gradient: 512 -> 320 on 96 x 96 58 / 62
+// against 82 / 77 us, two 640 -> 128 on 120 x 72 71 / 66 against 109 / 138, 320 -> 320 on 64 x 64 30 / 29 against 46 / 27;
+// two 128 -> 640 on 120 x 72 stay unfolded forward (73 against 65).
+enum class Direct { kNo, kExact, kRagged };
+Direct conv3_form(const ConvShape& g, at::ScalarType t, int64_t in_ch, int64_t out_ch, const at::Tensor& x, const at::Tensor& w,
+                  bool adjoint) {
   const char* off = std::getenv("VKT_CONV_IM2COL");
-  if (dptr(x) % 16 != 0 || dptr(w) % 16 != 0) return false;
-  return !(off != nullptr && off[0] == '1') && coop_is_enabled() && (t == at::kBFloat16 || t == at::kHalf) && g.KH == 3 && g.KW == 3 && g.SH == 1 &&
-         g.SW == 1 && g.PH == 1 && g.PW == 1 && in_ch % 16 == 0 && out_ch % 128 == 0 && g.W % 64 == 0 &&
-         g.N * g.H * (g.W / 64) * (out_ch / 128) <= 0x7fffffffLL;
+  if (dptr(x) % 16 != 0 || dptr(w) % 16 != 0) return Direct::kNo;
+  if ((off != nullptr && off[0] == '1') || !coop_is_enabled() || (t != at::kBFloat16 && t != at::kHalf) || g.KH != 3 || g.KW != 3 ||
+      g.SH != 1 || g.SW != 1 || g.PH != 1 || g.PW != 1 || in_ch % 16 != 0 || g.N * g.H * g.W * ((out_ch + 127) / 128) > 0x7fffffffLL)
+    return Direct::kNo;
+  if (out_ch % 128 == 0 && g.W % 64 == 0) return Direct::kExact;
+  if (out_ch % 32 != 0 || out_ch < 128 || g.W % 8 != 0) return Direct::kNo;
+  const int64_t S = hrt_conv3r_splits(g.N, in_ch, out_ch, g.H, g.W);
+  const int64_t tiles = g.N * ((g.H + 3) / 4) * ((g.W + 31) / 32) * ((out_ch + 127) / 128) * S;
+  const double px = (double)(g.N * g.H) * g.W, split = S > 1 ? 3.0 + 1.3e-6 * S * out_ch * px : 0.0;
+  const double direct = (double)((tiles + 255) / 256) * (1.6 * in_ch / 16 / S + 3.5) + 5.0 + split;
+  const double product = 18.0 * in_ch * out_ch * px / 600e6 + 6.0, columns = 18e-6 * g.C * px;  // us; MB
+  const double unfolded = product + (adjoint ? 4.0 + columns / 2.2 : 8.0 + columns / 2.8);
+  return 1.05 * direct < unfolded ? Direct::kRagged : Direct::kNo;
 }
 
 // y = conv3x3(x) with the weights reordered for the kernel (flip = 0: the forward, w [out_ch, in_ch, 3, 3];
 // flip = 1: the input gradient, w [in_ch, out_ch, 3, 3] read as its flipped transpose), plus bias.
 at::Tensor conv3_run(const at::Tensor& x, const at::Tensor& w, const at::Tensor* bias, const ConvShape& g,
-                     int64_t in_ch, int64_t out_ch, uint32_t flip) {
-  const at::Tensor wr = at::empty({hrt_conv3_wr_bytes(out_ch, in_ch) / 2}, x.options());
+                     int64_t in_ch, int64_t out_ch, uint32_t flip, Direct form) {
+  const bool rag = form == Direct::kRagged;
+  const int64_t wr_bytes = rag ? hrt_conv3r_wr_bytes(out_ch, in_ch) : hrt_conv3_wr_bytes(out_ch, in_ch);
+  const at::Tensor wr = at::empty({wr_bytes / 2}, x.options());
   hrt_conv3_wprep_args P{};
   P.w = dptr(w), P.wr = dptr(wr), P.O = out_ch, P.I = in_ch, P.flip = flip;
-  queue(typed("conv3x3_wprep", x.scalar_type()), P);
+  queue(typed(rag ? "conv3x3r_wprep" : "conv3x3_wprep", x.scalar_type()), P);
   at::Tensor y = at::empty({g.N, out_ch, g.H, g.W}, x.options());
-  const int64_t splits = hrt_conv3_splits(g.N, in_ch, out_ch, g.H, g.W);
+  const int64_t splits = rag ? hrt_conv3r_splits(g.N, in_ch, out_ch, g.H, g.W) : hrt_conv3_splits(g.N, in_ch, out_ch, g.H, g.W);
   at::Tensor ws;  // the splits' fp32 partial sums
   if (splits > 1) ws = at::empty({splits * g.N * out_ch * g.H * g.W}, x.options().dtype(at::kFloat));
   hrt_conv3_args A{};
   A.x = dptr(x), A.wr = dptr(wr), A.y = dptr(y), A.ws = splits > 1 ? dptr(ws) : 0;
   A.N = g.N, A.I = in_ch, A.O = out_ch, A.H = g.H, A.W = g.W, A.splits = (uint32_t)splits;
   if (bias) A.bias = dptr(*bias), A.has_bias = 1;
-  queue(typed("conv3x3", x.scalar_type()), A);
+  queue(typed(rag ? "conv3x3r" : "conv3x3", x.scalar_type()), A);
   note_gpu("torch_vulkan::conv3x3");  // lets callers and tests see which path ran
   return y;
 }
 
 // The weight matrix w2 [M, K] times each image's column matrix cols[n] [K, L] -> [N, M, L]: a plain GEMM for a
 // single image, else one batched GEMM whose left operand repeats w2 with a zero batch stride (no copy).
-at::Tensor weight_times(const at::Tensor& w2, const at::Tensor& cols) {
+at::Tensor weight_times(const at::Tensor& w2, const at::Tensor& cols, const at::Tensor* bias = nullptr) {
+  if (bias != nullptr) {  // added in fp32 by the product's epilogue (one bias value per row)
+    const at::Tensor b = bias->view({-1, 1});
+    if (cols.size(0) == 1) return at::addmm(b, w2, cols[0]).unsqueeze(0);
+    return at::baddbmm(b, w2.expand({cols.size(0), w2.size(0), w2.size(1)}), cols);
+  }
   if (cols.size(0) == 1) return at::mm(w2, cols[0]).unsqueeze(0);
   return at::bmm(w2.expand({cols.size(0), w2.size(0), w2.size(1)}), cols);
 }
@@ -134,15 +158,15 @@ at::Tensor k_convolution_overrideable(const at::Tensor& input, const at::Tensor&
   if (c && (!has_bias || (on_vk(*bias) && bias->scalar_type() == input.scalar_type() && bias->numel() == c->Co))) {
     const ConvShape& g = *c;
     const at::Tensor xd = dense(input), wd = dense(weight);
-    if (conv3_ok(g, input.scalar_type(), g.C, g.Co, xd, wd)) {
+    if (const Direct form = conv3_form(g, input.scalar_type(), g.C, g.Co, xd, wd, false); form != Direct::kNo) {
       const at::Tensor b = has_bias ? dense(*bias) : at::Tensor();
-      at::Tensor out = conv3_run(xd, wd, has_bias ? &b : nullptr, g, g.C, g.Co, 0);
+      at::Tensor out = conv3_run(xd, wd, has_bias ? &b : nullptr, g, g.C, g.Co, 0, form);
       note_gpu("aten::convolution_overrideable");
       return out;
     }
     at::Tensor cols = cols_of(input, g);
-    at::Tensor out = weight_times(wd.view({g.Co, g.K()}), cols).view({g.N, g.Co, g.OH, g.OW});
-    if (has_bias) out.add_(bias->view({1, g.Co, 1, 1}));
+    const at::Tensor b = has_bias ? dense(*bias) : at::Tensor();
+    at::Tensor out = weight_times(wd.view({g.Co, g.K()}), cols, has_bias ? &b : nullptr).view({g.N, g.Co, g.OH, g.OW});
     note_gpu("aten::convolution_overrideable");
     return out;
   }
@@ -177,8 +201,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> k_convolution_backward_overrideab
   const at::Tensor wd = dense(weight);
   at::Tensor w2 = wd.view({g.Co, g.K()});
   at::Tensor gi, gw, gb;
-  if (mask[0] && conv3_ok(g, go.scalar_type(), g.Co, g.C, go, wd)) {
-    gi = conv3_run(go, wd, nullptr, g, g.Co, g.C, 1);  // the adjoint: flipped, transposed kernel
+  const Direct form = mask[0] ? conv3_form(g, go.scalar_type(), g.Co, g.C, go, wd, true) : Direct::kNo;
+  if (form != Direct::kNo) {
+    gi = conv3_run(go, wd, nullptr, g, g.Co, g.C, 1, form);  // the adjoint: flipped, transposed kernel
   } else if (mask[0]) {
     at::Tensor gcols = dense(weight_times(w2.t(), G));  // [N, K, L]
     if (g.direct()) {
