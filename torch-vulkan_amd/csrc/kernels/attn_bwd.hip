@@ -733,7 +733,7 @@ constexpr int QST = 128;  // queries per LDS stage of the dK / dV kernel
 // PAD: as the forward's.  SPLIT: few key blocks (a 77-token context: two per head) would leave most CUs idle, so
 // `splits` workgroups share a key block, each taking a run of query stages and writing fp32 partial dK, dV
 // ([split][b h][key][2][D] in p.o32) that attn_dkdv_sum adds in split order (B2 H8, 1024 queries, 77 keys of 80: 56 us
-// on 32 workgroups of the general kernel; the whole forward + backward 88 -> 47).
+// on 32 workgroups of the general kernel; the whole forward + backward 88 -> 43).
 template <typename T, int DCH, bool PAD, bool SPLIT>
 __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb, int splits) {
   constexpr int NW = 8;
@@ -857,7 +857,7 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb, i
   //   P = exp2(acc_S sl2) = exp(scale S - lse),   -dS = P acc_dP = P (delta - dP).
   const float nis = -1.f / p.scale;
   auto stage = [&](auto bc, auto rc, int st) {
-    constexpr int BUF = decltype(bc)::value;
+    const int BUF = bc;  // a constant of the full stages
     constexpr bool RAGGED = decltype(rc)::value;
     const bool COPY = st + 1 < st1;
     const HK_L uint8_t* Qt = (BUF ? Q1 : Q0) + qq * 32 * ROWB;
@@ -999,12 +999,9 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb, i
     stage(I0(), std::false_type(), st);
     ++st;
   }
-  if (st < st1) {  // the ragged last stage, in buffer (st - st0) & 1
-    if ((st - st0) & 1)
-      stage(I1(), std::true_type(), st);
-    else
-      stage(I0(), std::true_type(), st);
-  }
+  // the ragged last stage: one instance for both buffers (two, joining after a branch, spilled 300 bytes a lane at
+  // D = 128: B4 H13 S1858 308 us)
+  if (st < st1) stage((st - st0) & 1, std::true_type(), st);
 
   // ---- sum the four query quarters of each key group, dK first, then dV.  Piece (k, n) = d block n of key
   // group k, finished by its owner wave (k, own(n)); the three other waves' partials go to slots 0..2 of
@@ -1120,15 +1117,17 @@ __global__ __launch_bounds__(256) void attn_dkdv_sum(hrt_attn_args p, int splits
 }
 
 // Query splits of the fast dK / dV path: as many as keep its workgroups within one round of 256, whole 128-query stages
-// each.  A split costs its partials' write and read and a launch (~6 us): only where the stages one workgroup
-// would walk take longer (from 3 on, at ~4 us a stage).
+// each.  A split costs its partials' write and read and a launch (5 - 7 us); a stage that a workgroup no longer walks
+// saves ~1.1 us in 128-wide tiles and ~0.8 in 64-wide ones.  Forward + backward unsplit / split: 588 keys of 128, B3 H1,
+// 896 queries (6 stages saved) 39.6 / 42.0 us, 1408 (10) 45.4 / 42.2, 2048 (15) 54.5 / 45.3; 77 keys of 80, B2 H8,
+// 1024 queries (7) 35.3 / 33.6; keys of 64, H8: 300 and 1024 queries (7) 31.7 / 33.2, 500 and 2048 (12) 40.4 / 36.1.
 int dkdv_splits(const hrt_attn_args& a) {
   const int64_t wgs = (int64_t)((a.Sk + 63) / 64) * a.B * a.H, nst = (a.Sq + QST - 1) / QST;
-  if (wgs > 128 || nst < 4) return 1;
+  if (wgs > 128) return 1;
   int64_t s = 256 / wgs;
   if (s > nst) s = nst;
   const int64_t per = cdiv(nst, s);
-  return (int)cdiv(nst, per);
+  return nst - per >= (a.D > 64 ? 7 : 10) ? (int)cdiv(nst, per) : 1;
 }
 
 // The direct-to-LDS paths need D % 8 == 0 above 32, 16-byte aligned rows (q, k, v, dout) and per-stage row
