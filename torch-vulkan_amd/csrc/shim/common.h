@@ -47,6 +47,15 @@ std::string typed(std::string_view op, at::ScalarType t);
 inline bool on_vk(const at::Tensor& t) { return t.defined() && t.device().type() == kDev; }
 inline uint64_t dptr(const at::Tensor& t) { return reinterpret_cast<uint64_t>(t.data_ptr()); }
 inline at::Tensor dense(const at::Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
+// Workspace that only makes an operator faster: n elements, or an undefined tensor where the memory limit, the device or
+// a graph being recorded has no room for it and the operator goes on without.
+inline at::Tensor scratch_or_none(int64_t n, const at::TensorOptions& o) {
+  try {
+    return at::empty({n}, o);
+  } catch (const c10::Error&) {
+    return {};
+  }
+}
 inline bool present(const std::optional<at::Tensor>& t) { return t.has_value() && t->defined(); }
 
 // ---- accounting -------------------------------------------------------------------------------------------

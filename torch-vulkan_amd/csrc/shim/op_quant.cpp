@@ -65,9 +65,9 @@ at::Tensor dequant_int8_linear_vk(const at::Tensor& x, const at::Tensor& q, cons
     A.bias = dptr(*bias), A.has_bias = 1;
   }
   at::Tensor deq;
-  if (hrt_mm_dq8_workspace(&A) > 0) {
-    deq = at::empty({N, K}, x.options());
-    A.ws = dptr(deq);
+  if (const int64_t ws = hrt_mm_dq8_workspace(&A); ws > 0) {
+    deq = scratch_or_none(ws, x.options());
+    if (deq.defined()) A.ws = dptr(deq);
   }
   queue(typed("mm_dq8", x.scalar_type()), A);
   note_gpu("torch_vulkan::dequant_int8_linear");
