@@ -371,9 +371,13 @@ double tile_us(const TileCost& c, TileShape sh, uint32_t tiles, uint32_t steps) 
   if (rest) us += first + out * fill + steps * last;
   return us;
 }
-// The partial products of a split: their write and read (at ~5 TB/s, a little of it lost to the tail of the slices)
-// and the second launch (1024 x 2048 x 8192, four slices: 10 us over the slices alone).
-double split_us(int64_t splits, int64_t M, int64_t N) { return 3.3 + 0.3 * splits + 1.1 * (double)splits * M * N * 4 / 5e6; }
+// The partial products of a split: their write and read (at ~6 TB/s, a little of it lost to the tail of the slices),
+// the second launch, and each slice's start (1024 x 2048 x 8192, four slices: 10 us over the slices alone).  Charged at
+// 4.5 TB/s, 1024 x 2048 x 6144 NN went to two slices of 128 x 128 tiles, 42.6 us with their sum, instead of four of
+// 128 x 256, 41.1 (a DiT block's forward and backward 678.2 -> 675.9 us, a
+// 951 x 4928 x 1472 linear layer 92.9 -> 83.8; 7522 x 4352 x 256, whose weight gradient went from three slices to six,
+// 131.6 -> 134.7).
+double split_us(int64_t splits, int64_t M, int64_t N) { return 3.3 + 0.33 * splits + 0.85 * (double)splits * M * N * 4 / 5e6; }
 
 struct GemmPlan {
   int tile = -1;  // GemmTile, -1: the direct-to-LDS kernel does not take the product
