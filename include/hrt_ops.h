@@ -194,7 +194,7 @@ int64_t hrt_mm_workspace(const hrt_mm_args* mm, int32_t dtype);
  * weights would otherwise be converted once per 256-row block of x) the weights are dequantized into it
  * once and the product runs on them; the values are the same either way.  For small M it may hold fp32 partial
  * products over slices of K, added in order (a reduction order of its own).  hrt_mm_dq8_workspace gives the
- * elements that help a call: N * K or 0. */
+ * elements that help a call: N * K, the size of those partial products (at most N * K), or 0. */
 typedef struct hrt_mm_dq8_args {
   uint64_t x, q, scale, bias, y;
   int64_t M, N, K, nblocks;

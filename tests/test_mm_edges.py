@@ -195,3 +195,19 @@ def test_split_plan_on_the_host():
     assert plan(128, 128, 4096, dtype=abi.F32) % (128 * 128) == 0 and plan(128, 128, 4096, dtype=abi.F32) > 0
     assert plan(2048, 2048, 64, dtype=abi.F32) == 0
     assert plan(604, 704, 5184, batch=2, a_sb=604 * 5184, b_sb=704 * 5184) == 0
+
+
+def test_int8_workspace_is_the_size_of_what_it_holds():
+    """Few rows: the fp32 partial products of 2 to 8 K slices, not the dequantized weights, whose 256 MiB at 16384 x
+    8192 would be a reservation from the driver and a wait for the GPU on every call (16 rows: 340 us, 138 without)."""
+    lib = ctypes.CDLL(abi._LIB_PATH)
+    lib.hrt_mm_dq8_workspace.restype = ctypes.c_int64
+
+    def elems(m, n, k):
+        p = abi.MmDq8Args(x=4096, q=8192, scale=4096, y=4096, M=m, N=n, K=k, nblocks=k // 64, x_sm=k, x_sk=1, alpha=1.0)
+        return lib.hrt_mm_dq8_workspace(ctypes.byref(p))
+
+    for m, n, k in [(1, 16384, 8192), (16, 16384, 8192), (16, 8192, 16384), (16, 8192, 2048), (100, 2048, 8192)]:
+        w = elems(m, n, k)
+        assert 0 < w <= n * k and w % (2 * m * n) == 0 and 2 <= w // (2 * m * n) <= 8, (m, n, k, w)
+    assert elems(4096, 8192, 2048) == 8192 * 2048 and elems(1024, 8192, 2048) == 0

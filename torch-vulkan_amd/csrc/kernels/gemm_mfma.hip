@@ -521,8 +521,8 @@ void queue_dq8(const hrt_mm_dq8_args& a, hipStream_t s) {
 }
 
 // The same choice for the fused int8 linear (tile costs include the conversion of the int8 tile: M = 512 at 8192 x 2048
-// weights 31 us on 128 x 128 tiles, 41 on 256 x 128, 50 on 64 x 64; M = 16 on 64 x 64 12 us in four slices, 19 unsplit).  A split keeps its partial products in the optional workspace, whose N K 16-bit
-// elements hold them while 2 splits M <= K.
+// weights 31 us on 128 x 128 tiles, 41 on 256 x 128, 50 on 64 x 64; M = 16 on 64 x 64 12 us in four slices, 19 unsplit).  A split keeps its partial products in the optional workspace, which a caller may size for the
+// dequantized weights: N K 16-bit elements hold them while 2 splits M <= K.
 GemmPlan plan_dq8(const hrt_mm_dq8_args& d, bool may_split) {
   static constexpr struct {
     GemmTile t;
@@ -765,5 +765,6 @@ extern "C" int64_t hrt_mm_workspace(const hrt_mm_args* a, int32_t dtype) {
 extern "C" int64_t hrt_mm_dq8_workspace(const hrt_mm_dq8_args* a) {
   if (a == nullptr || a->M <= 0 || a->N <= 0 || a->K <= 0) return 0;
   if (a->M >= hk::kDq8WsMinM) return a->N * a->K;
-  return hk::plan_dq8(*a, true).splits > 1 ? a->N * a->K : 0;
+  const int64_t splits = hk::plan_dq8(*a, true).splits;
+  return splits > 1 ? 2 * splits * a->M * a->N : 0;  // fp32 partial products in 16-bit elements
 }
