@@ -765,6 +765,7 @@ extern "C" int64_t hrt_mm_workspace(const hrt_mm_args* a, int32_t dtype) {
 extern "C" int64_t hrt_mm_dq8_workspace(const hrt_mm_dq8_args* a) {
   if (a == nullptr || a->M <= 0 || a->N <= 0 || a->K <= 0) return 0;
   if (a->M >= hk::kDq8WsMinM) return a->N * a->K;
+  // not N K: 256 MiB and more is a reservation and a wait for the GPU on every call (16 x 16384 x 8192 340 us, 41 so)
   const int64_t splits = hk::plan_dq8(*a, true).splits;
   return splits > 1 ? 2 * splits * a->M * a->N : 0;  // fp32 partial products in 16-bit elements
 }
