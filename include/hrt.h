@@ -68,7 +68,12 @@ void hrt_set_memory_limit(uint64_t bytes);
  * Replaces `vkrt_alloc` (csrc/vkrt.h:16). */
 uint64_t hrt_alloc(uint64_t size);
 
-/* Free an address returned by hrt_alloc.  Unknown addresses and double frees are rejected (-1).
+/* The same for workspace that a caller can do without: 0, with no error set, where the free ranges and one more slab
+ * have no room.  It never gives idle slabs back, never waits for the GPU and makes no dedicated slab; after a refused
+ * slab it asks the driver for none until memory came back.  Freed by hrt_free.  No counterpart in csrc/vkrt.h. */
+uint64_t hrt_alloc_spare(uint64_t size);
+
+/* Free an address returned by hrt_alloc or hrt_alloc_spare.  Unknown addresses and double frees are rejected (-1).
  * Replaces `vkrt_free` (csrc/vkrt.h:17). */
 int hrt_free(uint64_t addr);
 

@@ -14,9 +14,10 @@ struct FakeBacking : hrt::Backing {
   uint64_t next = 0x100000000ull;
   uint64_t capacity = ~0ull;  // bytes the "driver" can hand out
   uint64_t mapped = 0;
-  int drains = 0;
+  int drains = 0, maps = 0;
   std::map<uint64_t, uint64_t> live;
   bool map(uint64_t size, uint64_t* base, std::string* err) override {
+    ++maps;
     if (mapped + size > capacity) {
       *err = "fake out of memory";
       return false;
@@ -169,6 +170,41 @@ static int memory_limit_and_retry() {
   return 0;
 }
 
+// Workspace that can be done without: free ranges and whole regular slabs only; no idle slab given back, no drain, and
+// a refused slab not asked for again until memory came back.
+static int spare_blocks() {
+  FakeBacking fb;
+  fb.capacity = 1ull << 30;
+  hrt::SlabAllocator a(&fb, 288ull << 30);
+  std::string err;
+  uint64_t x = a.alloc_spare(100ull << 20);
+  CHECK(x && a.slab_count() == 1 && a.live_bytes() == 100ull << 20 && a.resolve(x, 100ull << 20, &err));
+  uint64_t y = a.alloc_spare(300ull << 20);  // above the dedicated threshold: still part of a regular slab
+  CHECK(y && a.slab_count() == 1 && a.is_regular_block(y));
+  uint64_t z = a.alloc(450ull << 20, &err);  // dedicated: the driver has 62 MiB left
+  CHECK(z && a.slab_count() == 2);
+  CHECK(a.free(x, &err) && a.free(y, &err));  // an idle slab, which a tensor's allocation would give back
+  const int drains = fb.drains;
+  fb.maps = 0;
+  for (int i = 0; i < 5; ++i) CHECK(a.alloc_spare(513ull << 20) == 0);
+  uint64_t whole = a.alloc_spare(512ull << 20);
+  CHECK(whole);
+  for (int i = 0; i < 5; ++i) CHECK(a.alloc_spare(1 << 20) == 0);
+  CHECK(fb.maps == 1 && fb.drains == drains && a.slab_count() == 2);
+  CHECK(a.free(z, &err));  // memory came back: asked for again
+  uint64_t w = a.alloc_spare(1 << 20);
+  CHECK(w && fb.maps == 2 && a.free(w, &err) && a.free(whole, &err));
+  CHECK(a.empty_cache() == 2 && fb.mapped == 0);
+  a.set_limit(64ull << 20);  // one slab of 64 MiB: a smaller one near the cap
+  uint64_t p = a.alloc(1 << 20, &err), q = a.alloc_spare(63ull << 20);
+  CHECK(p && q && a.alloc_spare(1 << 20) == 0 && a.slab_count() == 1);
+  CHECK(a.free(q, &err));
+  a.set_frozen(true);
+  q = a.alloc_spare(40ull << 20);
+  CHECK(q && a.alloc_spare(40ull << 20) == 0);
+  return 0;
+}
+
 static int peak_tracking() {
   FakeBacking fb;
   hrt::SlabAllocator a(&fb, 288ull << 30);
@@ -185,7 +221,7 @@ static int peak_tracking() {
 
 int main() {
   int (*tests[])() = {many_small_allocations, coalescing_and_isolation, no_merge_across_adjacent_slabs, bounds_and_double_free,
-                      dedicated_blocks_and_empty_cache, memory_limit_and_retry, peak_tracking};
+                      dedicated_blocks_and_empty_cache, memory_limit_and_retry, spare_blocks, peak_tracking};
   int fails = 0;
   for (auto t : tests) fails += t();
   printf(fails ? "FAILED\n" : "ALL OK\n");

@@ -414,6 +414,13 @@ uint64_t hrt_alloc(uint64_t size) {
   return a;
 }
 
+uint64_t hrt_alloc_spare(uint64_t size) {
+  Runtime* rt = rt_or_error();
+  if (!rt) return 0;
+  std::lock_guard<std::mutex> l(rt->mu);
+  return rt->alloc->alloc_spare(size);
+}
+
 int hrt_free(uint64_t addr) {
   Runtime* rt = rt_or_error();
   if (!rt) return -1;

@@ -67,6 +67,7 @@ class SlabAllocator {
 
   void set_limit(uint64_t bytes) {
     limit_ = bytes;
+    spare_refused_ = false;
     if (bytes > 0) {
       uint64_t s = bytes / 8;
       if (s > (256ull << 20)) s = 256ull << 20;
@@ -106,16 +107,8 @@ class SlabAllocator {
     } else {
       addr = carve(rounded);
       if (addr == 0) {
-        uint64_t want = slab_bytes_;
-        if (limit_ > 0) {
-          uint64_t res = reserved_bytes();
-          uint64_t head = limit_ > res ? limit_ - res : 0;
-          head -= head % kAlign;
-          if (head >= rounded && head < want) want = head;
-        }
-        if (want < rounded) want = rounded;
         uint64_t base = 0;
-        if (!new_slab_with_retry(want, /*dedicated=*/false, &base, err)) return 0;
+        if (!new_slab_with_retry(regular_slab_bytes(rounded), /*dedicated=*/false, &base, err)) return 0;
         addr = carve(rounded);
         if (addr == 0) {
           *err = "allocation failed right after creating a slab";
@@ -125,6 +118,27 @@ class SlabAllocator {
     }
     auto slab_it = slab_of(addr);
     blocks_[addr] = Block{rounded, size, slab_it->first};
+    live_ += rounded;
+    if (live_ > peak_) peak_ = live_;
+    return addr;
+  }
+
+  // A block for memory that an operator can do without, 0 where there is no room: from the free ranges, or from a new
+  // regular slab.  Unlike alloc() it gives no idle slab back to the driver, never waits for the GPU and makes no
+  // dedicated slab (which free() would drain the GPU for), and once a slab was refused asks for no other until memory
+  // came back or the cap changed.
+  uint64_t alloc_spare(uint64_t size) {
+    if (size == 0 || size > max_alloc_) return 0;
+    const uint64_t rounded = (size + kAlign - 1) / kAlign * kAlign;
+    uint64_t addr = carve(rounded);
+    if (addr == 0 && !frozen_ && !spare_refused_ && rounded <= slab_bytes_) {
+      uint64_t base = 0;
+      std::string err;
+      if (new_slab_checked(regular_slab_bytes(rounded), /*dedicated=*/false, &base, &err)) addr = carve(rounded);
+      else spare_refused_ = true;
+    }
+    if (addr == 0) return 0;
+    blocks_[addr] = Block{rounded, size, slab_of(addr)->first};
     live_ += rounded;
     if (live_ > peak_) peak_ = live_;
     return addr;
@@ -146,6 +160,7 @@ class SlabAllocator {
       backing_->drain();  // queued kernels may still read it
       backing_->unmap(sit->first);
       slabs_.erase(sit);
+      spare_refused_ = false;
       return true;
     }
     insert_free(blk.slab, addr, blk.size);
@@ -177,6 +192,7 @@ class SlabAllocator {
       it = slabs_.erase(it);
       ++n;
     }
+    if (n > 0) spare_refused_ = false;
     return n;
   }
 
@@ -281,6 +297,18 @@ class SlabAllocator {
     by_size_.insert({len, addr});
   }
 
+  // Size of the regular slab made for a block: a whole one, near the cap what is left of it.
+  uint64_t regular_slab_bytes(uint64_t rounded) const {
+    uint64_t want = slab_bytes_;
+    if (limit_ > 0) {
+      const uint64_t res = reserved_bytes();
+      uint64_t head = limit_ > res ? limit_ - res : 0;
+      head -= head % kAlign;
+      if (head >= rounded && head < want) want = head;
+    }
+    return want < rounded ? rounded : want;
+  }
+
   bool new_slab_checked(uint64_t size, bool dedicated, uint64_t* base, std::string* err) {
     if (limit_ > 0) {
       uint64_t res = reserved_bytes();
@@ -291,6 +319,7 @@ class SlabAllocator {
       }
     }
     if (!backing_->map(size, base, err)) return false;
+    spare_refused_ = false;
     Slab s;
     s.size = size;
     s.dedicated = dedicated;
@@ -315,6 +344,7 @@ class SlabAllocator {
   uint64_t max_alloc_;
   uint64_t limit_ = 0;
   bool frozen_ = false;
+  bool spare_refused_ = false;  // a slab for alloc_spare was refused, and no memory has come back since
   uint64_t slab_bytes_ = kSlabBytes;
   uint64_t dedicated_min_ = kDedicatedMin;
   uint64_t live_ = 0, peak_ = 0;

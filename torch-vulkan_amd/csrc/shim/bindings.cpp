@@ -100,6 +100,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fallback_counts", &cpu_counts);
   m.def("fallback_time_by_op", &cpu_seconds_by_op);
   m.def("reset_counts", &clear_counts);
+  m.def("workspaces_left_out", &vkt::scratch_left_out);
   m.def("runtime_counters", [] {
     runtime();
     std::vector<uint64_t> c;

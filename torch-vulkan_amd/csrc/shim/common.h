@@ -47,15 +47,13 @@ std::string typed(std::string_view op, at::ScalarType t);
 inline bool on_vk(const at::Tensor& t) { return t.defined() && t.device().type() == kDev; }
 inline uint64_t dptr(const at::Tensor& t) { return reinterpret_cast<uint64_t>(t.data_ptr()); }
 inline at::Tensor dense(const at::Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
-// Workspace that only makes an operator faster: n elements, or an undefined tensor where the memory limit, the device or
-// a graph being recorded has no room for it and the operator goes on without.
-inline at::Tensor scratch_or_none(int64_t n, const at::TensorOptions& o) {
-  try {
-    return at::empty({n}, o);
-  } catch (const c10::Error&) {
-    return {};
-  }
-}
+// Workspace that only makes an operator faster: `bytes` of device memory until the handle goes (kernels queued before
+// may still use it: one stream), or an empty handle where there is no room and the operator goes on without; every
+// empty one is counted.  By default (hrt_alloc_spare) nothing is given up for it: no idle slab, no wait for the GPU.
+// reserve: room is made as for a tensor.
+c10::DataPtr scratch(int64_t bytes, bool reserve = false);
+inline uint64_t dptr(const c10::DataPtr& p) { return reinterpret_cast<uint64_t>(p.get()); }
+uint64_t scratch_left_out();  // how many were empty
 inline bool present(const std::optional<at::Tensor>& t) { return t.has_value() && t->defined(); }
 
 // ---- accounting -------------------------------------------------------------------------------------------

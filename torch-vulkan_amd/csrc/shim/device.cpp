@@ -18,6 +18,7 @@
 #include <c10/core/impl/DeviceGuardImplInterface.h>
 
 #include <array>
+#include <atomic>
 #include <cstring>
 #include <mutex>
 #include <shared_mutex>
@@ -146,6 +147,8 @@ class PinnedMemory final : public c10::Allocator {
 
 DeviceMemory g_device_memory;
 PinnedMemory g_pinned_memory;
+
+std::atomic<uint64_t> g_scratch_left_out{0};
 
 // Give a storage `nbytes` bytes, keeping the leading min(old, new) bytes of its contents.  The new block
 // is filled on the device (queued copy), then swapped in; the old block is freed when its DataPtr dies.
@@ -286,6 +289,14 @@ void copy_between(const at::Tensor& dst, const at::Tensor& src, bool non_blockin
 namespace vkt {
 c10::Allocator* device_allocator() { return &g_device_memory; }
 c10::Allocator* pinned_allocator() { return &g_pinned_memory; }
+
+c10::DataPtr scratch(int64_t bytes, bool reserve) {
+  runtime();
+  const uint64_t a = reserve ? hrt_alloc(static_cast<uint64_t>(bytes)) : hrt_alloc_spare(static_cast<uint64_t>(bytes));
+  if (a == 0) ++g_scratch_left_out;
+  return wrap(a, &DeviceMemory::release, c10::Device(kDev, 0));
+}
+uint64_t scratch_left_out() { return g_scratch_left_out.load(); }
 }  // namespace vkt
 
 namespace {

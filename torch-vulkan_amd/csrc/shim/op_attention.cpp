@@ -218,10 +218,10 @@ BwdOut k_sdpa_bwd(const at::Tensor& grad_out, const at::Tensor& query, const at:
     hrt_attn_args KV = A;
     KV.dk = dptr(dk);
     KV.dv = dptr(dv);
-    at::Tensor partial;  // few key blocks: partial dK, dV of query ranges
+    c10::DataPtr partial;  // few key blocks: partial dK, dV of query ranges
     if (const int64_t ws = matrix_cores(dt) ? hrt_attn_dkdv_workspace(&KV) : 0; ws > 0) {
-      partial = scratch_or_none(ws, q.options().dtype(at::kFloat));
-      if (partial.defined()) KV.o32 = dptr(partial), KV.flags |= HRT_ATTN_DKDV_WS;
+      partial = scratch(ws * 4);
+      if (partial) KV.o32 = dptr(partial), KV.flags |= HRT_ATTN_DKDV_WS;
     }
     queue(attn_kernel("dkdv", dt), KV);
     note_gpu(kBwdOp);

@@ -194,7 +194,7 @@ std::optional<at::Tensor> try_product(const at::Tensor& a, const at::Tensor& b, 
   hrt_mm_args A = p->args;
   A.c = dptr(out);
   const int64_t ws = (matrix_cores || p->dt == at::kFloat) && !p->batched ? hrt_mm_workspace(&A, float_code(p->dt)) : 0;
-  if (const at::Tensor partial = ws > 0 ? scratch_or_none(ws, out.options().dtype(at::kFloat)) : at::Tensor(); partial.defined()) {
+  if (const c10::DataPtr partial = ws > 0 ? scratch(ws * 4) : c10::DataPtr(); partial) {
     const hrt_mm_splitk_args X{A, dptr(partial), ws};
     queue(typed("mm_splitk", p->dt), X);
   } else {

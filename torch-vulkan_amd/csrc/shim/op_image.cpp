@@ -126,9 +126,9 @@ at::Tensor conv3_run(const at::Tensor& x, const at::Tensor& w, const at::Tensor*
   queue(typed(rag ? "conv3x3r_wprep" : "conv3x3_wprep", x.scalar_type()), P);
   at::Tensor y = at::empty({g.N, out_ch, g.H, g.W}, x.options());
   int64_t splits = rag ? hrt_conv3r_splits(g.N, in_ch, out_ch, g.H, g.W) : hrt_conv3_splits(g.N, in_ch, out_ch, g.H, g.W);
-  at::Tensor ws;  // the splits' fp32 partial sums
-  if (splits > 1) ws = scratch_or_none(splits * g.N * out_ch * g.H * g.W, x.options().dtype(at::kFloat));
-  if (!ws.defined()) splits = 1;
+  c10::DataPtr ws;  // the splits' fp32 partial sums
+  if (splits > 1) ws = scratch(splits * g.N * out_ch * g.H * g.W * 4);
+  if (!ws) splits = 1;
   hrt_conv3_args A{};
   A.x = dptr(x), A.wr = dptr(wr), A.y = dptr(y), A.ws = splits > 1 ? dptr(ws) : 0;
   A.N = g.N, A.I = in_ch, A.O = out_ch, A.H = g.H, A.W = g.W, A.splits = (uint32_t)splits;

@@ -64,10 +64,10 @@ at::Tensor dequant_int8_linear_vk(const at::Tensor& x, const at::Tensor& q, cons
                 "dequant_int8_linear: bias must be a contiguous vk tensor of ", N, " elements in x's dtype");
     A.bias = dptr(*bias), A.has_bias = 1;
   }
-  at::Tensor deq;
-  if (const int64_t ws = hrt_mm_dq8_workspace(&A); ws > 0) {
-    deq = scratch_or_none(ws, x.options());
-    if (deq.defined()) A.ws = dptr(deq);
+  c10::DataPtr ws;
+  if (const int64_t n = hrt_mm_dq8_workspace(&A); n > 0) {
+    ws = scratch(n * 2, /*reserve=*/M >= 2048);  // the weights once, for many rows, repay a reservation
+    if (ws) A.ws = dptr(ws);
   }
   queue(typed("mm_dq8", x.scalar_type()), A);
   note_gpu("torch_vulkan::dequant_int8_linear");

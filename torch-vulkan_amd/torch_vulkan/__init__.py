@@ -114,6 +114,12 @@ def slab_count() -> int:
     return _C.slab_count()
 
 
+def workspaces_left_out() -> int:
+    """How often an operator ran without a workspace that would have made it faster, for want of device memory; the
+    last bits of its result then differ (another order of fp32 sums)."""
+    return _C.workspaces_left_out()
+
+
 def manual_seed(seed: int) -> None:
     # random numbers are drawn on the CPU and copied, as in the reference
     return None

@@ -187,6 +187,7 @@ class Runtime:
             "hrt_reset_peak_live_bytes": (None, []),
             "hrt_set_memory_limit": (None, [u64]),
             "hrt_alloc": (u64, [u64]),
+            "hrt_alloc_spare": (u64, [u64]),
             "hrt_free": (ctypes.c_int, [u64]),
             "hrt_upload": (ctypes.c_int, [u64, vp, u64]),
             "hrt_download": (ctypes.c_int, [vp, u64, u64]),
