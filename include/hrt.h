@@ -172,7 +172,8 @@ float hrt_event_elapsed_ms(uint32_t start_slot, uint32_t end_slot);
  * graph instead of being executed; calls that would wait for the GPU (upload, download, synchronize,
  * freeing a dedicated block, empty_cache) and allocations that need a new slab fail while recording.
  * hrt_graph_end returns the graph id (>= 0, -1 on error); hrt_graph_launch queues one replay on the
- * runtime stream (asynchronous), hrt_graph_destroy releases it. */
+ * runtime stream (asynchronous), hrt_graph_destroy releases it.  Memory freed while recording (operators'
+ * intermediates and workspaces, which every replay writes) stays with the graph until it is destroyed. */
 int hrt_graph_begin(void);
 int64_t hrt_graph_end(void);
 int hrt_graph_launch(int64_t graph);

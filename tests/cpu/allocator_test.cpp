@@ -205,6 +205,41 @@ static int spare_blocks() {
   return 0;
 }
 
+// Ranges held for a recorded graph: given to nobody, their slab not idle, until released.
+static int held_ranges() {
+  FakeBacking fb;
+  hrt::SlabAllocator a(&fb, 288ull << 30);
+  std::string err;
+  std::vector<hrt::SlabAllocator::Piece> held, none;
+  uint64_t x = a.alloc(4096, &err), y = a.alloc(8192, &err), z = a.alloc(4096, &err);
+  CHECK(a.free(x, &err) && a.free(y, &err));
+  uint64_t u = a.alloc(512, &err);  // a live block inside what x and y had
+  CHECK(u == x);
+  a.hold(x, 4096, &held);
+  a.hold(y, 8192, &held);
+  a.hold(y, 4096, &held);  // held already: no second piece
+  a.hold(z, 4096, &none);  // live: nothing to hold
+  uint64_t sum = 0;
+  for (const auto& p : held) sum += p.len;
+  CHECK(sum == 4096 + 8192 - 512 && none.empty());
+  for (int i = 0; i < 100; ++i) {
+    const uint64_t v = a.alloc(512 << (i % 6), &err);
+    CHECK(v && (v >= z + 4096 || v + (512ull << (i % 6)) <= x));
+  }
+  CHECK(a.free(u, &err));
+  CHECK(a.alloc(512, &err) == u);  // a live block's range is its own again once freed
+  CHECK(a.free(u, &err) && a.free(z, &err));
+  hrt::SlabAllocator b(&fb, 288ull << 30);
+  held.clear();
+  x = b.alloc(4096, &err);
+  CHECK(b.free(x, &err));
+  b.hold(x, 4096, &held);
+  CHECK(held.size() == 1 && b.empty_cache() == 0);
+  b.release(held);
+  CHECK(b.empty_cache() == 1);
+  return 0;
+}
+
 static int peak_tracking() {
   FakeBacking fb;
   hrt::SlabAllocator a(&fb, 288ull << 30);
@@ -221,7 +256,7 @@ static int peak_tracking() {
 
 int main() {
   int (*tests[])() = {many_small_allocations, coalescing_and_isolation, no_merge_across_adjacent_slabs, bounds_and_double_free,
-                      dedicated_blocks_and_empty_cache, memory_limit_and_retry, spare_blocks, peak_tracking};
+                      dedicated_blocks_and_empty_cache, memory_limit_and_retry, spare_blocks, held_ranges, peak_tracking};
   int fails = 0;
   for (auto t : tests) fails += t();
   printf(fails ? "FAILED\n" : "ALL OK\n");

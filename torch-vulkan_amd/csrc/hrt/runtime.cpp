@@ -91,7 +91,12 @@ struct Runtime {
   hipEvent_t prof_ev[2] = {nullptr, nullptr};
   static constexpr uint32_t kSlots = 1024;  // timing events (hrt_event_record)
   hipEvent_t slots[kSlots] = {};
-  std::vector<hipGraphExec_t> graphs;
+  struct Graph {
+    hipGraphExec_t exec = nullptr;
+    std::vector<SlabAllocator::Piece> held;  // memory of intermediates: every replay writes it
+  };
+  std::vector<Graph> graphs;
+  std::vector<std::pair<uint64_t, uint64_t>> freed_recording;  // blocks freed while a graph is being recorded
   // Asynchronous uploads run on their own stream (default priority) so they overlap kernels.
   hipStream_t copy_stream = nullptr;
   hipEvent_t order_ev = nullptr;      // compute-stream position an upload starts after
@@ -431,6 +436,7 @@ int hrt_free(uint64_t addr) {
     set_error("hrt_free: a dedicated block cannot be released while a graph is being recorded");
     return -1;
   }
+  if (rt->backing.capturing) rt->freed_recording.emplace_back(addr, rt->alloc->block_bytes(addr));
   if (!rt->alloc->free(addr, &err)) {
     set_error(err);
     return -1;
@@ -794,6 +800,7 @@ int hrt_graph_begin(void) {
   if (e != hipSuccess) return hip_fail("hipStreamBeginCapture", e);
   rt->backing.capturing = true;
   rt->alloc->set_frozen(true);
+  rt->freed_recording.clear();
   return 0;
 }
 
@@ -816,7 +823,13 @@ int64_t hrt_graph_end(void) {
   e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
   if (e != hipSuccess) return hip_fail("hipGraphInstantiate", e);
-  rt->graphs.push_back(x);
+  // Within the recording, memory that one operator freed (workspaces, intermediates) served the next, in stream order.
+  // From here on it is the graph's: given to a later tensor, a replay would overwrite it.
+  Runtime::Graph rec;
+  rec.exec = x;
+  for (const auto& [addr, len] : rt->freed_recording) rt->alloc->hold(addr, len, &rec.held);
+  rt->freed_recording.clear();
+  rt->graphs.push_back(std::move(rec));
   return (int64_t)rt->graphs.size() - 1;
 }
 
@@ -824,7 +837,7 @@ int hrt_graph_launch(int64_t graph) {
   Runtime* rt = rt_or_error();
   if (!rt) return -1;
   std::lock_guard<std::mutex> l(rt->mu);
-  if (graph < 0 || graph >= (int64_t)rt->graphs.size() || !rt->graphs[graph]) {
+  if (graph < 0 || graph >= (int64_t)rt->graphs.size() || !rt->graphs[graph].exec) {
     set_error("hrt_graph_launch: unknown graph id");
     return -1;
   }
@@ -832,7 +845,7 @@ int hrt_graph_launch(int64_t graph) {
     set_error("hrt_graph_launch: not allowed while a graph is being recorded");
     return -1;
   }
-  hipError_t e = hipGraphLaunch(rt->graphs[graph], rt->stream);
+  hipError_t e = hipGraphLaunch(rt->graphs[graph].exec, rt->stream);
   if (e != hipSuccess) return hip_fail("hipGraphLaunch", e);
   return 0;
 }
@@ -841,13 +854,14 @@ int hrt_graph_destroy(int64_t graph) {
   Runtime* rt = rt_or_error();
   if (!rt) return -1;
   std::lock_guard<std::mutex> l(rt->mu);
-  if (graph < 0 || graph >= (int64_t)rt->graphs.size() || !rt->graphs[graph]) {
+  if (graph < 0 || graph >= (int64_t)rt->graphs.size() || !rt->graphs[graph].exec) {
     set_error("hrt_graph_destroy: unknown graph id");
     return -1;
   }
   (void)hipStreamSynchronize(rt->stream);
-  (void)hipGraphExecDestroy(rt->graphs[graph]);
-  rt->graphs[graph] = nullptr;
+  (void)hipGraphExecDestroy(rt->graphs[graph].exec);
+  rt->alloc->release(rt->graphs[graph].held);
+  rt->graphs[graph] = {};
   return 0;
 }
 

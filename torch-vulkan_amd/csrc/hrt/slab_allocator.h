@@ -28,6 +28,7 @@
 #include <set>
 #include <string>
 #include <utility>
+#include <vector>
 
 namespace hrt {
 
@@ -165,6 +166,34 @@ class SlabAllocator {
     }
     insert_free(blk.slab, addr, blk.size);
     return true;
+  }
+
+  // Ranges that nothing else may be given although no block is live in them: what is free of [addr, addr + len) leaves
+  // the free ranges (and keeps its slab from being idle) until release() of the pieces appended to *held.
+  struct Piece {
+    uint64_t addr, len, slab;
+  };
+  void hold(uint64_t addr, uint64_t len, std::vector<Piece>* held) {
+    auto it = free_.upper_bound(addr);
+    if (it != free_.begin()) --it;
+    while (it != free_.end() && it->first < addr + len) {
+      const uint64_t lo = it->first, hi = lo + it->second.len, slab = it->second.slab;
+      const uint64_t a = lo > addr ? lo : addr, b = hi < addr + len ? hi : addr + len;
+      ++it;
+      if (a >= b) continue;
+      by_size_.erase({hi - lo, lo});
+      free_.erase(lo);
+      if (a > lo) insert_free(slab, lo, a - lo);
+      if (hi > b) insert_free(slab, b, hi - b);
+      slabs_[slab].used += b - a;
+      held->push_back({a, b - a, slab});
+    }
+  }
+  void release(const std::vector<Piece>& held) {
+    for (const Piece& p : held) {
+      slabs_[p.slab].used -= p.len;
+      insert_free(p.slab, p.addr, p.len);
+    }
   }
 
   // Return every slab without live blocks; returns how many were released.
