@@ -428,7 +428,7 @@ __global__ __launch_bounds__(512) void attn_fwd_dma(hrt_attn_args p, int nqb) {
     qf[ks] = *reinterpret_cast<const HK_L u32x4*>(V1 + tile_off<NCH>(g * 32 + ql, 2 * ks + hl));
   f32x16 sa = qk(K0), sb;
   mask_and_max(sa, 0);
-  __syncthreads();  // every wave is done with K(0) and Q before they are copied over
+  barrier_keep_vm_lds<0>();  // K(1) landed; every wave is done with K(0) and Q before they are copied over
   using M2 = std::integral_constant<int, 2>;
   using M1 = std::integral_constant<int, 1>;
   using M0 = std::integral_constant<int, 0>;

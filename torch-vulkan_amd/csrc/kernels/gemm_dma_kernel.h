@@ -253,7 +253,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void mm_dma(hrt_mm_args
     for (int c = 0; c < IPA; ++c) copy_a(0, A0, c);
 #pragma unroll
     for (int c = 0; c < IPB; ++c) copy_b(0, B0, c);
-    __syncthreads();
+    barrier_keep_vm_lds<0>();
   } else if constexpr (!DQ8) {
     // steps 0 .. RING - 2 into buffers 0 .. RING - 2 (step min(s, nk - 1): a short K re-copies its last step
     // into buffers nobody reads)
@@ -285,7 +285,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void mm_dma(hrt_mm_args
     barrier_keep_vm<IPA + 2 * IPQ>();  // int8 step 0 and A step 0 landed everywhere
     dq_scales(k1, svq);
     dq_convert(Q0, B0, sv);
-    __syncthreads();  // B tile 0 written; the other copies landed
+    barrier_keep_vm_lds<0>();  // B tile 0 written; the other copies landed
   }
 
   // K step kt: MFMAs from buffer kt % 3, copies of step min(kt + 2, nk - 1) into buffer (kt + 2) % 3 (read
@@ -384,7 +384,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void mm_dma(hrt_mm_args
         if (fly == F || (F == RING - 2 && fly > F)) barrier_keep_vm<F * (IPA + IPB)>();
       });
     } else {
-      __syncthreads();  // the next step's copies, issued in this one, have landed everywhere
+      barrier_keep_vm_lds<0>();  // the next step's copies, issued in this one, have landed everywhere
     }
   };
   using I0 = std::integral_constant<int, 0>;
@@ -420,7 +420,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void mm_dma(hrt_mm_args
       if (kt + 6 >= nk) break;
     }
   }
-  __syncthreads();  // the last copies have landed before the epilogue reuses the tiles
+  __syncthreads();  // (the last step waited for its copies) the epilogue reuses the tiles
 
   // ---- epilogue: per n sub-tile j, the WM x 32 fp32 block goes through this wavefront's area as [m][n]
   float* const area = reinterpret_cast<float*>(wave < PA            ? a0_raw + wave * AREA

@@ -244,7 +244,9 @@ __device__ __forceinline__ u32x2 lds_tr4(const HK_L uint8_t* p) {
 
 // Workgroup barrier that lets the N most recently issued vector-memory operations of this wavefront (the
 // copies of a later stage) stay in flight: waits until at most N are outstanding, then joins the barrier.
-// __syncthreads() would wait for all of them (its release fence waits for every outstanding load).  The
+// __syncthreads() says nothing about copies into LDS: the compiler waits for them where the same wavefront reads what
+// they wrote, which publishes nothing to the others, and it has left the wait out before barriers on a loop's back
+// edge.  Every barrier that publishes copies is therefore one of these two, N = 0 where none may stay in flight.  The
 // wait is the s_waitcnt builtin (vmcnt in bits 3:0 and 15:14, expcnt 7 and lgkmcnt 15 = no wait), which
 // the compiler's wait-insertion pass takes into account: reads of a stage whose copies it has seen
 // complete get no further wait.  The barrier is an asm statement with a memory clobber, so the compiler
