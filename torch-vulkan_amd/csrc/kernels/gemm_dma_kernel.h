@@ -121,6 +121,11 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void mm_dma(hrt_mm_args
     tm = (sub / nbn) * (uint32_t)xbm + loc / bnw;
     tn = (sub % nbn) * bnw + loc % bnw;
   }
+  if constexpr (EDGE) {
+    // the divisions leave these in vector registers, and with them every address computed from them; a buffer resource
+    // built there is wrapped in a loop over the lanes at each copy (ten instructions and a branch, between the MFMAs)
+    tm = __builtin_amdgcn_readfirstlane(tm), tn = __builtin_amdgcn_readfirstlane(tn), bz = __builtin_amdgcn_readfirstlane(bz);
+  }
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
   // this workgroup's K range: all of it, or slice bz of a product split along K
   int64_t k0 = 0;
