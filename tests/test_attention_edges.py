@@ -91,3 +91,16 @@ def test_few_keys_share_out_the_queries(B, H, Sq, Sk, D):
 @pytest.mark.parametrize("pad,offset", [(8, 8), (4, 4), (5, 3)])
 def test_16_bit_alignments(pad, offset):
     check(1, 2, 300, 200, 80, torch.float16, REL16[torch.float16], pad, offset)
+
+
+@pytest.mark.parametrize("dt,B,H,D", [(torch.float32, 4097, 4096, 1), (torch.float16, 2049, 4096, 40)])
+def test_more_workgroups_than_one_launch_holds(dt, B, H, D):
+    """More (batch, head) pairs than workgroups of 256 (f32) or 512 threads fit below 2^32 work items: kernels of fewer
+    threads take them, and the last pairs are there as well.  One key: o = v, dv = do, dq = dk = 0."""
+    q = torch.ones(1, dtype=dt, device=dev).expand(B * H * D).contiguous().view(B, H, 1, D).requires_grad_(True)
+    v = torch.full((1,), 3.0, dtype=dt, device=dev).expand(B * H * D).contiguous().view(B, H, 1, D).requires_grad_(True)
+    out = F.scaled_dot_product_attention(q, q, v)
+    dq, dv = torch.autograd.grad(out, (q, v), v.detach())
+    for t, want in ((out, 3.0), (dv, 3.0), (dq, 0.0)):
+        for i in (0, 2047, B - 2, B - 1):
+            assert torch.equal(t[i].detach().cpu(), torch.full((H, 1, D), want, dtype=dt)), (i, want)

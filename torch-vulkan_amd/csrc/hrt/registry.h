@@ -90,6 +90,10 @@ inline uint64_t span_bytes(int ndim, const int64_t* sizes, const int64_t* stride
   return (last + 1) * elem;
 }
 
+// Whether a one-dimensional launch runs all of its workgroups: from 2^32 work items on, HIP starts only some of them and
+// reports no error.
+inline bool grid_fits(int64_t blocks, int64_t threads) { return blocks * threads < (int64_t(1) << 32); }
+
 inline bool launch_ok(hipError_t e, LaunchCtx& ctx, const char* what) {
   if (e == hipSuccess) return true;
   ctx.error = std::string(what) + ": " + hipGetErrorString(e);

@@ -1145,9 +1145,9 @@ bool launch_dkdv(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   if (!attn_check(a, false, true, false, 2, ctx)) return false;
   const int nkb = (a.Sk + 63) / 64;
   const int64_t total = (int64_t)nkb * a.B * a.H;
-  if (total > 0x7fffffffLL) return ctx.fail("grid too large");
+  if (!hrt::grid_fits(total, 256)) return ctx.fail("grid too large");
   const dim3 g((uint32_t)total);
-  if (bwd_dma_ok(a)) {
+  if (bwd_dma_ok(a) && hrt::grid_fits(total, 512)) {
     const int64_t part = (int64_t)a.B * a.H * a.Sk * 2 * a.D;  // floats of one split's partials
     const int splits = (a.flags & HRT_ATTN_DKDV_WS) && a.o32 % 16 == 0 ? dkdv_splits(a) : 1;
     if (splits > 1 && !ctx.check(a.o32, (uint64_t)(part * splits) * 4, "o32")) return false;
@@ -1189,11 +1189,11 @@ bool launch_dq(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   if (!attn_check(a, false, false, true, 2, ctx)) return false;
   const int nqb = (a.Sq + 63) / 64;
   const int64_t total = (int64_t)nqb * a.B * a.H;
-  if (total > 0x7fffffffLL) return ctx.fail("grid too large");
+  if (!hrt::grid_fits(total, 256)) return ctx.fail("grid too large");
   const bool with_delta = (a.flags & HRT_ATTN_DQ_DELTA) != 0;
   const bool of32 = (a.flags & HRT_ATTN_O_F32) != 0;
   const dim3 g((uint32_t)total);
-  if (bwd_dma_ok(a)) {
+  if (bwd_dma_ok(a) && hrt::grid_fits(total, 512)) {
     if (with_delta && !ctx.check(a.o, (uint64_t)a.B * a.H * a.Sq * a.D * (of32 ? 4 : 2), "o")) return false;
 #define HK_DQ(DCH, PAD)                                                                                     \
   if (!with_delta)                                                                                          \

@@ -215,8 +215,8 @@ bool launch_fma(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   if (!attn_check(a, W == 0, W == 1, W == 2, sizeof(typename T::storage), ctx)) return false;
   const int nb = ((W == 1 ? a.Sk : a.Sq) + 63) / 64;
   const int64_t total = (int64_t)nb * a.B * a.H;
-  if (total > 0x7fffffffLL) return ctx.fail("grid too large");
-  if constexpr (std::is_same<T, F32>::value)  // the fp32 matrix cores, unless their 31-bit offsets do not reach
+  if (!hrt::grid_fits(total, 64)) return ctx.fail("grid too large");
+  if constexpr (std::is_same<T, F32>::value)  // the fp32 matrix cores, unless their 31-bit offsets or their grid do not reach
     if (attn_f32_mfma(a, W, ctx.stream)) return hrt::launch_ok(hipGetLastError(), ctx, "attn_f32_mfma");
   const dim3 g((uint32_t)total);
   const int dch = (a.D + 31) / 32;

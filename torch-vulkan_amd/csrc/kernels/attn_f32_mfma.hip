@@ -363,8 +363,10 @@ void queue_d(const hrt_attn_args& a, hipStream_t s) {
 
 }  // namespace
 
-// Queues the kernel (0 forward, 1 dK/dV, 2 dQ); false (nothing queued) when a stage's offsets do not fit 31 bits.
+// Queues the kernel (0 forward, 1 dK/dV, 2 dQ); false (nothing queued) when a stage's offsets do not fit 31 bits or the
+// grid is too large (the scalar kernels take 64 rows in 64 threads, these 32 in 256).
 bool attn_f32_mfma(const hrt_attn_args& a, int which, hipStream_t s) {
+  if (!hrt::grid_fits(cdiv(which == 1 ? a.Sk : a.Sq, 32) * a.B * a.H, 256)) return false;
   const int64_t lim = ((int64_t)1 << 31) / (4 * 130);
   if (a.q_ss >= lim || a.k_ss >= lim || a.v_ss >= lim || (which != 0 && a.do_ss >= lim)) return false;
   // 16-byte accesses: whole 16-byte chunks of d, rows of every operand and output on 16-byte lines

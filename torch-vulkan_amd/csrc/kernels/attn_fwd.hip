@@ -548,9 +548,9 @@ bool launch_fwd(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   if (!attn_check(a, true, false, false, 2, ctx)) return false;
   const int nqb = (a.Sq + 63) / 64;
   const int64_t total = (int64_t)nqb * a.B * a.H;
-  if (total > 0x7fffffffLL) return ctx.fail("grid too large");
+  if (!hrt::grid_fits(total, 256)) return ctx.fail("grid too large");
   const dim3 g((uint32_t)total);
-  if (fwd_dma_ok(a)) {
+  if (fwd_dma_ok(a) && hrt::grid_fits(total, 512)) {
     // 65 to 96 columns pay for 128: the 96-wide rows of the general kernel's tiles have no copy swizzle, and it is
     // slower all the same (forward + backward at B1 H4 S1395 D80: 170 us there, 59 on padded tiles)
     if (a.D == 128) hipLaunchKernelGGL((attn_fwd_dma<T, 4, false>), g, dim3(512), 0, ctx.stream, a, nqb);
