@@ -104,3 +104,26 @@ def test_more_workgroups_than_one_launch_holds(dt, B, H, D):
     for t, want in ((out, 3.0), (dv, 3.0), (dq, 0.0)):
         for i in (0, 2047, B - 2, B - 1):
             assert torch.equal(t[i].detach().cpu(), torch.full((H, 1, D), want, dtype=dt)), (i, want)
+
+
+@pytest.mark.parametrize("D,dt", [(40, torch.bfloat16), (56, torch.float16), (80, torch.float16), (96, torch.bfloat16), (120, torch.float16),
+                                  (64, torch.float32), (80, torch.float32)])
+@pytest.mark.parametrize("Sq,Sk", [(200, 300), (300, 200), (130, 130), (60, 50), (1100, 60)])
+def test_infinities_and_nans_reach_their_column(Sq, Sk, D, dt):
+    """An infinity or NaN of v (of the output's gradient) reaches its own column of o (of dv) and nothing else, also from
+    a row that a partial last stage copies a second time and masks (zero times infinity would be NaN)."""
+    g = torch.Generator().manual_seed(Sq + D)
+    q, k, v, go = (torch.randn((1, 2, s, D), generator=g).to(dt) for s in (Sq, Sk, Sk, Sq))
+    for s, t in ((Sk, v), (Sq, go)):
+        t[0, 0, s - 5, 3] = float("inf")
+        t[0, 1, s // 2, D - 1] = float("nan")
+        if s > 128:
+            t[0, 0, (s - 1) // 128 * 128 - 3, 7] = -float("inf")  # in the stage before the last
+    leaves = [t.to(dev).requires_grad_(True) for t in (q, k, v)]
+    o = F.scaled_dot_product_attention(*leaves)
+    dv = torch.autograd.grad(o, leaves, go.to(dev))[2]
+    P = torch.softmax(q.double() @ k.double().transpose(-1, -2) / math.sqrt(D), -1)
+    for got, want in ((o, P @ v.double()), (dv, P.transpose(-1, -2) @ go.double())):
+        got = got.detach().cpu()
+        for f in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(f(got), f(want)), f

@@ -817,7 +817,7 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb, i
     const int valid = SPLIT ? (int)(Sq - org) : Sq;
     if constexpr (PAD) {
       edge_tile<NCH, QST, NW>(Qb + org * qss, qss, valid, dch, Q0, wave, lane);
-      edge_tile<NCH, QST, NW>(Ob + org * oss, oss, valid, dch, O0, wave, lane);
+      edge_tile<NCH, QST, NW>(Ob + org * oss, oss, valid, dch, O0, wave, lane, repeated_rows<QST>(st0, nst, Sq));
     } else {
       dma_tile<NCH, QST, NW>(Qb + org * qss, qss, valid, Q0, wave, lane, dma_lane_offsets<NCH>(qss, lane, j0));
       dma_tile<NCH, QST, NW>(Ob + org * oss, oss, valid, O0, wave, lane, dma_lane_offsets<NCH>(oss, lane, j0));
@@ -882,7 +882,9 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb, i
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int qa = org + qq * 32 + 8 * j + 4 * hl + r;
-          s[4 * j + r] = qa >= st * QST && qa < Sq ? s[4 * j + r] : -INFINITY;
+          const bool in = qa >= st * QST && qa < Sq;
+          s[4 * j + r] = in ? s[4 * j + r] : -INFINITY;
+          if (PAD) dp[4 * j + r] = in ? dp[4 * j + r] : 0.f;
         }
     }
     const HK_G uint8_t* const qn = Qb + stage_origin<QST>(st + 1, nst, Sq) * qss;
@@ -903,12 +905,13 @@ __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb, i
       const int rsub = ln / NCH;
       const uint32_t x0 = (uint32_t)(((ln % NCH) ^ tile_swz<NCH>(rsub)) << 4);
       const uint32_t bq = (uint32_t)rsub * qss, bo = (uint32_t)rsub * oss;
+      const int rep = PAD ? repeated_rows<QST>(st + 1, nst, Sq) - j0 * RPI - rsub : 0;  // dO rows copied as zeros
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const uint32_t x = x0 ^ (uint32_t)(tile_swz<NCH>(i * RPI) << 4);
         const bool in = !PAD || (int)(x >> 4) < dch;
         qlo.off[i] = in ? bq + x : kNoRow;
-        olo.off[i] = in ? bo + x : kNoRow;
+        olo.off[i] = in && (!PAD || i * RPI >= rep) ? bo + x : kNoRow;
       }
     }
     // S and dP products of d step ks; their operands (Q, dO, V rows) are read RA1 steps ahead into a ring,

@@ -372,6 +372,8 @@ __global__ __launch_bounds__(512) void attn_fwd_dma(hrt_attn_args p, int nqb) {
       const HK_G uint8_t* const vn = Vb + stage_origin<KST>(st + 1, nst, Sk) * vss;
       const __amdgpu_buffer_rsrc_t krs = PAD ? edge_rsrc(kn) : dma_rsrc(kn);
       const __amdgpu_buffer_rsrc_t vrs = PAD ? edge_rsrc(vn) : dma_rsrc(vn);
+      static_assert(IPW <= 4, "one lane offset per copy");
+      const DmaLanes vl = PAD && MODE == 1 ? edge_rows<NCH>(vlo, lane, j0, repeated_rows<KST>(st + 1, nst, Sk)) : vlo;
       // S(st+1) with this iteration's copies placed after its MFMAs, one per MFMA, then P(st); the VALU
       // work of P(st) is interleaved with the MFMAs by sched_group_barrier
       const HK_L uint8_t* Kt = BUF ? K0 : K1;
@@ -383,7 +385,7 @@ __global__ __launch_bounds__(512) void attn_fwd_dma(hrt_attn_args p, int nqb) {
       for (int ks = 0; ks < 2 * DCH; ++ks) {
         sn = Mfma32<T>::mac(kfr[ks], qf[ks], sn);
         if (ks < NK) dma_tile_part_rs<NCH, KST, NW>(krs, kss, BUF ? K1 : K0, wave, klo, ks);
-        else if (ks < NK + IPW) dma_tile_part_rs<NCH, KST, NW>(vrs, vss, BUF ? V0 : V1, wave, vlo, ks - NK);
+        else if (ks < NK + IPW) dma_tile_part_rs<NCH, KST, NW>(vrs, vss, BUF ? V0 : V1, wave, vl, ks - NK);
       }
 #pragma unroll
       for (int e = 0; e < 16; ++e) {

@@ -195,14 +195,14 @@ __device__ __forceinline__ void edge_copy(__amdgpu_buffer_rsrc_t rs, HK_L uint8_
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, tile + j * 1024, 16, (int)off, 0, 0, 0);
 }
 
-// A ROWS x NCH-chunk tile whose rows hold only c_hi chunks (the rest reads zeros) and whose rows [valid, ROWS) are zeros,
-// copied by NW wavefronts.
+// A ROWS x NCH-chunk tile whose rows hold only c_hi chunks (the rest reads zeros) and whose rows [0, row_lo) and
+// [valid, ROWS) are zeros, copied by NW wavefronts.
 template <int NCH, int ROWS, int NW>
 __device__ __forceinline__ void edge_tile(const HK_G uint8_t* src, uint32_t ss, int valid, int c_hi, HK_L uint8_t* tile, int wave,
-                                          int lane) {
+                                          int lane, int row_lo = 0) {
   constexpr int IPW = ROWS * NCH / 64 / NW;
   uint32_t off[IPW];
-  edge_lane_offsets<NCH, IPW>(off, ss, lane, wave * IPW, 0, valid < ROWS ? valid : ROWS, 0, c_hi);
+  edge_lane_offsets<NCH, IPW>(off, ss, lane, wave * IPW, row_lo, valid < ROWS ? valid : ROWS, 0, c_hi);
   const __amdgpu_buffer_rsrc_t rs = edge_rsrc(src);
 #pragma unroll
   for (int i = 0; i < IPW; ++i) edge_copy(rs, tile, wave * IPW + i, off[i]);
@@ -217,6 +217,15 @@ __device__ __forceinline__ DmaLanes edge_lanes(uint32_t ss, int lane, int j0, in
   return d;
 }
 
+// `d` with the lanes of tile rows below row_lo masked as well.
+template <int NCH>
+__device__ __forceinline__ DmaLanes edge_rows(DmaLanes d, int lane, int j0, int row_lo) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if ((j0 + i) * (64 / NCH) + lane / NCH < row_lo) d.off[i] = kNoRow;
+  return d;
+}
+
 // First row of the tile that stage st copies when the sequence has more than one stage (len > ROWS): stage
 // st covers rows [st ROWS, (st + 1) ROWS); the last, ragged stage copies the full window that ends at row
 // len - 1 instead (origin len - ROWS), so no copy reads past the sequence, and its rows below st ROWS
@@ -226,6 +235,12 @@ __device__ __forceinline__ int64_t stage_origin(int st, int nst, int64_t len) {
   const int s = st < nst ? st : nst - 1;
   const int64_t o = (int64_t)s * ROWS;
   return o + ROWS <= len ? o : len - ROWS;
+}
+// Its rows that the stage before it has had: masked, their weights P are exact zeros, but a zero times an infinity among
+// them is NaN, so the padded forms copy zeros for the operand that P multiplies.
+template <int ROWS>
+__device__ __forceinline__ int repeated_rows(int st, int nst, int64_t len) {
+  return st == nst - 1 && nst > 1 && len % ROWS != 0 ? ROWS - (int)(len % ROWS) : 0;
 }
 
 // 16 bytes of a swizzled tile at (row, chunk c), as a byte offset.
