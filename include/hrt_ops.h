@@ -184,6 +184,21 @@ typedef struct hrt_mm_splitk_args {
  * are not aligned as the split kernel needs).  A pure host function of the sizes, strides and alignments. */
 int64_t hrt_mm_workspace(const hrt_mm_args* mm, int32_t dtype);
 
+/* Which kernel a product goes to and how it is cut up, for tests and tools.  Pure host functions of the sizes, strides and
+ * alignments, as the launches decide.  may_split: as "mm_splitk_*" with a workspace; with_ws: as "mm_dq8_*" with one. */
+enum {
+  HRT_MM_GENERAL = 0, /* 16 bits: register-staged tiles, any strides; f32: scalar FMA */
+  HRT_MM_DIRECT = 1,  /* operands copied straight to LDS, matrix cores (f32: any strides) */
+  HRT_MM_NARROW = 2,  /* kernels of their own for K <= 32 and for M or N <= 16 */
+  HRT_MM_DEQUANT = 3  /* int8: weights dequantized into the workspace, then HRT_MM_DIRECT */
+};
+typedef struct hrt_mm_plan {
+  int32_t kernel, tile_m, tile_n;
+  int32_t whole; /* 1: every tile and K step is whole, the form without masks */
+  int64_t splits;
+} hrt_mm_plan;
+int hrt_mm_plan_of(const hrt_mm_args* mm, int32_t dtype, int32_t may_split, hrt_mm_plan* plan);
+
 /* "mm_dq8_{bf16,f16}" — fused int8 weight-only linear (no reference counterpart; composes
  * csrc/ops_quant.cpp:34-59 with csrc/ops_mm.cpp:61-175):
  *   y[m, n] = alpha * sum_k x[m, k] * deq(q)[n, k] + beta * bias[n]
@@ -204,6 +219,7 @@ typedef struct hrt_mm_dq8_args {
   uint64_t ws;
 } hrt_mm_dq8_args;
 int64_t hrt_mm_dq8_workspace(const hrt_mm_dq8_args* args);
+int hrt_mm_dq8_plan_of(const hrt_mm_dq8_args* args, int32_t with_ws, hrt_mm_plan* plan);
 
 /* Fused scaled-dot-product attention, non-causal, no mask, D <= 128 (vkrt/shaders/attn.comp.in:1-14,
  * attn_coop.comp.in:1-9).  q: [B, H, Sq, D], k, v: [B, H, Sk, D] views given by (batch, head, seq)

@@ -9,6 +9,7 @@ terms' size, under 1e-5 here), then rounded once: relative L2 below the output's
 
 import ctypes
 import os
+import random
 
 import pytest
 import torch
@@ -180,6 +181,29 @@ def plan(m, n, k, a_off=0, dtype=abi.BF16, **kw):
     for name, v in kw.items():
         setattr(p, name, v)
     return lib.hrt_mm_workspace(ctypes.byref(p), dtype)
+
+
+def plan_of(m, n, k, ta=False, tb=True, dtype=abi.BF16, split=True, off=0):
+    """hrt_mm_plan_of for contiguous operands (ta: A stored [k][m], tb: B stored [n][k])."""
+    lib = ctypes.CDLL(abi._LIB_PATH)
+    p = abi.MmArgs(a=4096 + off, b=8192, c=1 << 20, M=m, N=n, K=k, batch=1, a_sm=1 if ta else k, a_sk=m if ta else 1,
+                   b_sk=1 if tb else n, b_sn=k if tb else 1, c_sm=n, c_sn=1, alpha=1.0)
+    out = abi.MmPlan()
+    assert lib.hrt_mm_plan_of(ctypes.byref(p), dtype, int(split), ctypes.byref(out)) == 0
+    return out
+
+
+def test_plan_query_agrees_with_the_workspace():
+    rng = random.Random(0)
+    for _ in range(300):
+        m, n, k = (rng.choice((rng.randint(1, 4000), 64 * rng.randint(1, 64))) for _ in range(3))
+        p = plan_of(m, n, k, tb=True)
+        w = plan(m, n, k)
+        assert (p.kernel == abi.MM_GENERAL) == (w < 0) and max(w, 0) == (p.splits * m * n if p.splits > 1 else 0), (m, n, k)
+        assert not p.whole or (m % p.tile_m == 0 and n % p.tile_n == 0 and k % 64 == 0)
+        assert p.kernel != abi.MM_NARROW or min(m, n) <= 16 or k <= 32
+        assert plan_of(m, n, k, split=False).splits == 1
+    assert plan_of(64, 64, 64, off=2).kernel == abi.MM_GENERAL
 
 
 def test_split_plan_on_the_host():

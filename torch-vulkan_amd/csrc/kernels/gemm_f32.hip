@@ -330,6 +330,12 @@ bool mm_f32_mfma(const hrt_mm_args& a, hipStream_t s) {
   return true;
 }
 
+void mm_f32_plan(const hrt_mm_args& a, bool may_split, hrt_mm_plan* out) {
+  if (!f32_fits(a)) return;
+  const bool whole = a.M % FT == 0 && a.N % FT == 0 && a.K % FBK == 0;
+  *out = hrt_mm_plan{HRT_MM_DIRECT, FT, FT, whole ? 1 : 0, may_split ? f32_splits(a) : 1};
+}
+
 int64_t mm_f32_workspace(const hrt_mm_args& a) {
   const int64_t s = f32_splits(a);
   return s > 1 ? s * a.M * a.N : 0;

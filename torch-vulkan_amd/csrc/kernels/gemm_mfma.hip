@@ -30,6 +30,7 @@ namespace hk {
 
 bool mm_check_operands(const hrt_mm_args& a, uint64_t elem, hrt::LaunchCtx& ctx);
 int64_t mm_f32_workspace(const hrt_mm_args& a);  // gemm_f32.hip
+void mm_f32_plan(const hrt_mm_args& a, bool may_split, hrt_mm_plan* out);
 
 namespace {
 
@@ -548,6 +549,19 @@ GemmPlan plan_dq8(const hrt_mm_dq8_args& d, bool may_split) {
   return best;
 }
 
+void fill_plan(const hrt_mm_args& a, const GemmPlan& p, hrt_mm_plan* out) {
+  if (p.tile < 0) return;
+  const TileShape t = kTileShape[p.tile];
+  *out = hrt_mm_plan{HRT_MM_DIRECT, t.bm, t.bn, dma_form(a, t.bm, t.bn).exact ? 1 : 0, p.splits};
+}
+
+// The product of a dequantize-first call: its B is the workspace (16-byte aligned).
+hrt_mm_args dq8_weights_as_mm(const hrt_mm_dq8_args& d) {
+  hrt_mm_args m = dq8_as_mm(d);
+  m.b = d.ws;
+  return m;
+}
+
 // Smallest M at which the fused int8 linear dequantizes into the caller's workspace first: the fused kernel
 // converts every weight once per 256-row block of x, which costs more than one standalone dequant pass
 // beyond a few blocks (M = 4096: 222 us fused vs ~157 us dequant + GEMM for 8192 x 2048 weights).
@@ -568,8 +582,7 @@ bool launch_mm_dq8(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
   // large M with a workspace: dequantize once (the dq8 kernel), then the fast GEMM on the bf16 / f16 weights
   const bool ws_ok = a.ws && a.ws % 16 == 0;
   if (ws_ok && a.M >= kDq8WsMinM && a.K % GBK == 0) {
-    hrt_mm_args m = dq8_as_mm(a);
-    m.b = a.ws;
+    const hrt_mm_args m = dq8_weights_as_mm(a);
     const GemmPlan plan = plan_gemm(m, false);
     if (plan.tile >= 0) {
       if (!ctx.check(a.ws, (uint64_t)(a.N * a.K) * 2, "ws")) return false;
@@ -768,4 +781,36 @@ extern "C" int64_t hrt_mm_dq8_workspace(const hrt_mm_dq8_args* a) {
   // not N K: 256 MiB and more is a reservation and a wait for the GPU on every call (16 x 16384 x 8192 340 us, 41 so)
   const int64_t splits = hk::plan_dq8(*a, true).splits;
   return splits > 1 ? 2 * splits * a->M * a->N : 0;  // fp32 partial products in 16-bit elements
+}
+
+// Both plans: 0, or -1 for a product that the launches refuse.
+extern "C" int hrt_mm_plan_of(const hrt_mm_args* a, int32_t dtype, int32_t may_split, hrt_mm_plan* out) {
+  if (a == nullptr || out == nullptr || a->M <= 0 || a->N <= 0 || a->K <= 0 || a->batch <= 0) return -1;
+  *out = hrt_mm_plan{HRT_MM_GENERAL, 64, 64, 0, 1};
+  if (dtype == HRT_F32) {
+    hk::mm_f32_plan(*a, may_split != 0, out);
+    return 0;
+  }
+  if (dtype != HRT_BF16 && dtype != HRT_F16) return -1;
+  if (hk::own_kernel(*a)) {
+    out->kernel = HRT_MM_NARROW;
+    return 0;
+  }
+  hk::fill_plan(*a, hk::plan_gemm(*a, may_split != 0), out);
+  return 0;
+}
+
+extern "C" int hrt_mm_dq8_plan_of(const hrt_mm_dq8_args* a, int32_t with_ws, hrt_mm_plan* out) {
+  if (a == nullptr || out == nullptr || a->M <= 0 || a->N <= 0 || a->K <= 0) return -1;
+  *out = hrt_mm_plan{HRT_MM_GENERAL, 64, 64, 0, 1};
+  if (with_ws != 0 && a->M >= hk::kDq8WsMinM && a->K % hk::GBK == 0) {
+    const hrt_mm_args m = hk::dq8_weights_as_mm(*a);
+    hk::fill_plan(m, hk::plan_gemm(m, false), out);
+    if (out->kernel == HRT_MM_DIRECT) {
+      out->kernel = HRT_MM_DEQUANT;
+      return 0;
+    }
+  }
+  hk::fill_plan(hk::dq8_as_mm(*a), hk::plan_dq8(*a, with_ws != 0), out);
+  return 0;
 }

@@ -119,6 +119,13 @@ class MmSplitkArgs(ctypes.Structure):
     _fields_ = [("mm", MmArgs), ("ws", u64), ("ws_floats", i64)]
 
 
+MM_GENERAL, MM_DIRECT, MM_NARROW, MM_DEQUANT = range(4)
+
+
+class MmPlan(ctypes.Structure):
+    _fields_ = [("kernel", i32), ("tile_m", i32), ("tile_n", i32), ("whole", i32), ("splits", i64)]
+
+
 class MmReduceArgs(ctypes.Structure):
     _fields_ = [("ws", u64), ("c", u64), ("bias", u64), ("M", i64), ("N", i64), ("splits", i64), ("c_sm", i64),
                 ("c_sn", i64), ("bias_sm", i64), ("bias_sn", i64), ("alpha", f32), ("beta", f32), ("has_bias", u32),
