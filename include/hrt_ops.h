@@ -139,7 +139,7 @@ typedef struct hrt_ew_args {
   int64_t c_strides[HRT_MAX_DIMS];
 } hrt_ew_args;
 
-/* "mm_{f32,bf16,f16}" (f32: the fp32 matrix cores; bf16, f16: portable FMA kernel) and "mm_mfma_{bf16,f16}" (gfx950 matrix cores):
+/* "mm_{f32,bf16,f16}" (f32: the fp32 matrix cores, for short K scalar FMA; bf16, f16: portable FMA kernel) and "mm_mfma_{bf16,f16}" (gfx950 matrix cores):
  *   c[b, m, n] = alpha * sum_k a[b, m, k] * b[b, k, n] + beta * bias[b, m, n]     (bias only if has_bias)
  * a, b, bias: any non-negative strides (transposed / sliced views are read in place; bias broadcasts
  * with stride 0); c: written with strides c_s*.  fp32 accumulation, one rounding at the store.

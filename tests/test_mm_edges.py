@@ -145,6 +145,30 @@ def test_f32_products(m, n, k, offset, ta, tb):
     assert ((out - want).norm() / want.norm()).item() <= 2 * tol
 
 
+# (m, n, k, batch, scalar): both sides of the lines between the scalar kernel and the matrix cores: 16-byte rows K = 16,
+# many narrow tiles 48; 4-byte copies 48, many narrow tiles 80, a batch of mostly empty ones 144
+F32_SHORT = [(100, 100, 16, 1, True), (100, 100, 20, 1, False), (64, 64, 1, 1, True), (101, 99, 47, 1, True), (101, 99, 49, 1, False),
+             (50000, 16, 48, 1, True), (50000, 16, 52, 1, False), (50001, 3, 79, 1, True), (50001, 3, 81, 1, False),
+             (3, 5, 143, 1000, True), (3, 5, 145, 1000, False), (7, 33, 79, 1000, True), (8, 32, 52, 1000, False)]
+
+
+@pytest.mark.parametrize("m,n,k,batch,scalar", F32_SHORT)
+def test_short_f32_reductions_stay_scalar(m, n, k, batch, scalar):
+    p = plan_of(m, n, k, dtype=abi.F32, batch=batch)
+    assert p.kernel == (abi.MM_GENERAL if scalar else abi.MM_DIRECT) and p.splits == 1
+
+
+@gpu
+@pytest.mark.parametrize("m,n,k,batch,scalar", F32_SHORT)
+def test_short_f32_reductions(m, n, k, batch, scalar):
+    g = torch.Generator().manual_seed(m + k)
+    a, b = torch.randn((batch, m, k), generator=g), torch.randn((batch, n, k), generator=g)
+    ref = a.double() @ b.double().transpose(1, 2)
+    A, B = a.to(dev), b.to(dev).transpose(1, 2)
+    out = (torch.bmm(A, B) if batch > 1 else torch.mm(A[0], B[0])).cpu().view(ref.shape)
+    assert ((out - ref).norm() / ref.norm()).item() <= 2.0**-23 * k**0.5 + 2.0**-23
+
+
 @gpu
 def test_f32_strided_batches_and_small_values():
     g = torch.Generator().manual_seed(0)
@@ -183,11 +207,11 @@ def plan(m, n, k, a_off=0, dtype=abi.BF16, **kw):
     return lib.hrt_mm_workspace(ctypes.byref(p), dtype)
 
 
-def plan_of(m, n, k, ta=False, tb=True, dtype=abi.BF16, split=True, off=0):
+def plan_of(m, n, k, ta=False, tb=True, dtype=abi.BF16, split=True, off=0, batch=1):
     """hrt_mm_plan_of for contiguous operands (ta: A stored [k][m], tb: B stored [n][k])."""
     lib = ctypes.CDLL(abi._LIB_PATH)
-    p = abi.MmArgs(a=4096 + off, b=8192, c=1 << 20, M=m, N=n, K=k, batch=1, a_sm=1 if ta else k, a_sk=m if ta else 1,
-                   b_sk=1 if tb else n, b_sn=k if tb else 1, c_sm=n, c_sn=1, alpha=1.0)
+    p = abi.MmArgs(a=4096 + off, b=8192, c=1 << 20, M=m, N=n, K=k, batch=batch, a_sm=1 if ta else k, a_sk=m if ta else 1,
+                   b_sk=1 if tb else n, b_sn=k if tb else 1, c_sm=n, c_sn=1, alpha=1.0, a_sb=m * k, b_sb=n * k, c_sb=m * n)
     out = abi.MmPlan()
     assert lib.hrt_mm_plan_of(ctypes.byref(p), dtype, int(split), ctypes.byref(out)) == 0
     return out

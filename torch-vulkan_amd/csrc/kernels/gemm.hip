@@ -11,6 +11,7 @@
 namespace hk {
 
 bool mm_f32_mfma(const hrt_mm_args& a, hipStream_t s);  // gemm_f32.hip
+bool mm_f32_scalar(const hrt_mm_args& a);
 
 namespace {
 
@@ -113,8 +114,8 @@ bool launch_mm_fma(const void* p, const uint32_t*, hrt::LaunchCtx& ctx) {
   const auto& a = *static_cast<const hrt_mm_args*>(p);
   if (a.flags != 0) return ctx.fail("the FMA GEMM takes no flags");
   if (!mm_check_operands(a, sizeof(typename T::storage), ctx)) return false;
-  if constexpr (std::is_same<T, F32>::value)  // the fp32 matrix cores, unless its 31-bit offsets do not reach
-    if (mm_f32_mfma(a, ctx.stream)) return hrt::launch_ok(hipGetLastError(), ctx, "mm_f32_dma");
+  if constexpr (std::is_same<T, F32>::value)  // the fp32 matrix cores, unless K is short or 31-bit offsets do not reach
+    if (!mm_f32_scalar(a) && mm_f32_mfma(a, ctx.stream)) return hrt::launch_ok(hipGetLastError(), ctx, "mm_f32_dma");
   if (cdiv(a.M, BM) > 65535) return ctx.fail("M too large for the FMA kernel grid");
   const dim3 grid((uint32_t)cdiv(a.N, BN), (uint32_t)cdiv(a.M, BM), (uint32_t)a.batch);
   hipLaunchKernelGGL(mm_fma<T>, grid, dim3(256), 0, ctx.stream, a);

@@ -1,5 +1,5 @@
-// fp32 products on the fp32 matrix cores: "mm_f32" wherever an operand tile's offsets fit 31 bits (gemm.hip keeps the
-// rest).  c = alpha * a @ b + beta * bias, fp32 multiplies and fp32 accumulation throughout (v_mfma_f32_32x32x2_f32:
+// fp32 products on the fp32 matrix cores: "mm_f32" wherever an operand tile's offsets fit 31 bits and the reduction is
+// not a short one (gemm.hip keeps the rest).  c = alpha * a @ b + beta * bias, fp32 multiplies and fp32 accumulation throughout (v_mfma_f32_32x32x2_f32:
 // no rounding of the inputs), as the scalar kernel it replaces and vkrt/shaders/mm.comp.in:90-154.
 //
 // Bound: the fp32 matrix rate (157 TFLOP/s published; 64 cycles per 32 x 32 x 2 MFMA and SIMD).  A 64 x 64 x 32 step of
@@ -224,17 +224,36 @@ bool f32_fits(const hrt_mm_args& a) {
          cdiv(a.M, FT) * cdiv(a.N, FT) * a.batch < lim;
 }
 
-void queue_mm_f32(const hrt_mm_args& a, int64_t kslice, hipStream_t s) {
-  // staged along the contiguous axis; 16-byte copies where every row (and batch entry) starts on a 16-byte line and
-  // holds whole chunks
+// Staged along the contiguous axis; 16-byte copies where every row (and batch entry) starts on a 16-byte line and holds
+// whole chunks.
+struct F32Form {
+  bool atr, btr, w16;
+};
+F32Form f32_form(const hrt_mm_args& a) {
   const bool atr = a.a_sm == 1 && a.a_sk != 1, btr = a.b_sn == 1 && a.b_sk != 1;
   const auto chunks = [&](uint64_t p, int64_t sb, bool tr, int64_t s_r, int64_t s_k, int64_t rows) {
     return p % 16 == 0 && (a.batch == 1 || sb % 4 == 0) &&
            (tr ? s_k % 4 == 0 && rows % 4 == 0 : s_k == 1 && s_r % 4 == 0 && a.K % 4 == 0);
   };
-  const bool w16 = chunks(a.a, a.a_sb, atr, a.a_sm, a.a_sk, a.M) && chunks(a.b, a.b_sb, btr, a.b_sn, a.b_sk, a.N);
-  if (w16) queue_f32<64, 64, 32, 32, true>(a, atr, btr, kslice, s);
-  else queue_f32<64, 64, 32, 32, false>(a, atr, btr, kslice, s);
+  return {atr, btr, chunks(a.a, a.a_sb, atr, a.a_sm, a.a_sk, a.M) && chunks(a.b, a.b_sb, btr, a.b_sn, a.b_sk, a.N)};
+}
+
+void queue_mm_f32(const hrt_mm_args& a, int64_t kslice, hipStream_t s) {
+  const F32Form f = f32_form(a);
+  if (f.w16) queue_f32<64, 64, 32, 32, true>(a, f.atr, f.btr, kslice, s);
+  else queue_f32<64, 64, 32, 32, false>(a, f.atr, f.btr, kslice, s);
+}
+
+// Short reductions stay on the scalar kernel (gemm.hip): it steps by 16 of K and its small workgroups share a CU, where
+// a tile here takes whole 32-float steps and the first loads of a deep ring.  Scalar against here, us: 100 x 100 x 16
+// 4.4 / 5.4, x 20 equal; 4-byte copies 101 x 99 x 33 6.6 / 7.0, x 49 8.0 / 7.0.  Many tiles mostly past the edge of a
+// narrow output last longer: 100000 x 3 x 16 9.3 / 18.7, 60000 x 16 x 48 0.90 of the time here, x 56 1.03; 4-byte copies
+// 100001 x 3 x 65 0.85, x 81 1.1; batches of 16384 3 x 5 x 129 0.93, of 1000 15 x 17 x 129 1.03.
+bool f32_scalar(const hrt_mm_args& a) {
+  if (a.K > 144 || cdiv(a.M, FT) > 65535) return false;
+  const bool narrow = a.M < a.N ? a.M <= 32 : a.N <= 32, many = cdiv(a.M, FT) * cdiv(a.N, FT) * a.batch >= 768;
+  if (f32_form(a).w16) return a.K <= (narrow && many ? 48 : 16);
+  return a.K <= (!narrow || !many ? 48 : a.M <= 32 && a.N <= 32 ? 144 : 80);
 }
 
 // K slices of one product (1: none): where its 64 x 64 tiles leave CUs idle.  A 32-float step of a tile takes 0.45 us of
@@ -323,6 +342,8 @@ HRT_REGISTER("mm_splitk_f32", hrt_mm_splitk_args, launch_mm_splitk_f32);
 
 }  // namespace
 
+bool mm_f32_scalar(const hrt_mm_args& a) { return f32_scalar(a); }
+
 // Queues the product; false (nothing queued) when a tile's element offsets do not fit 31 bits.
 bool mm_f32_mfma(const hrt_mm_args& a, hipStream_t s) {
   if (!f32_fits(a)) return false;
@@ -331,7 +352,7 @@ bool mm_f32_mfma(const hrt_mm_args& a, hipStream_t s) {
 }
 
 void mm_f32_plan(const hrt_mm_args& a, bool may_split, hrt_mm_plan* out) {
-  if (!f32_fits(a)) return;
+  if (!f32_fits(a) || f32_scalar(a)) return;
   const bool whole = a.M % FT == 0 && a.N % FT == 0 && a.K % FBK == 0;
   *out = hrt_mm_plan{HRT_MM_DIRECT, FT, FT, whole ? 1 : 0, may_split ? f32_splits(a) : 1};
 }
