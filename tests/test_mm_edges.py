@@ -88,6 +88,25 @@ def test_odd_reduction_of_m_and_n_contiguous_operands(k, ta, tb):
 
 
 @gpu
+@pytest.mark.parametrize("m,n,k,ld,dispatches", [(1024, 2048, 8192, 8194, 2), (1024, 2048, 6144, 6145, 2), (2048, 1536, 4096, 4097, 2),
+                                                 (256, 512, 6144, 6145, 1), (128, 256, 8192, 8200, 1)])
+def test_long_reductions_of_unaligned_operands_are_split(m, n, k, ld, dispatches):
+    """Rows off 16-byte lines: the general kernel over K slices, then their ordered sum; few blocks stay whole, aligned
+    rows (the last) go to mm_splitk, slices and sum in one dispatch."""
+    dt = torch.bfloat16
+    g = torch.Generator().manual_seed(ld)
+    a, b = torch.randn((m, k), generator=g).to(dt), torch.randn((n, k), generator=g).to(dt)
+    wide = torch.full((m, ld), float("nan"), dtype=dt)
+    wide[:, :k] = a
+    A, B = wide.to(dev)[:, :k], b.to(dev).t()
+    torch.vk.synchronize()
+    n0 = torch_vulkan.stats()["dispatch_n"]
+    out = torch.mm(A, B)
+    assert torch_vulkan.stats()["dispatch_n"] - n0 == dispatches
+    check(out, a.double() @ b.double().t(), dt)
+
+
+@gpu
 @pytest.mark.parametrize("m,n,k", [(130, 136, 72), (257, 264, 136)])
 def test_ragged_batches(m, n, k):
     dt = torch.float16

@@ -124,6 +124,9 @@ std::optional<Plan> plan(const at::Tensor& a, const at::Tensor& b, const at::Ten
 //  * other narrow products, one 64-wide output tile across (min(M, N) <= 64), whose operands are not 16-byte
 //    aligned: S doubles while the grid of 64 x 64 tiles stays within one workgroup per CU (256) and every
 //    slice keeps >= 128 of K.
+//  * wide products of such operands in whole 128 x 256 (256 x 128) blocks, fewer than 192 of them: S doubles until
+//    S x blocks >= 192 while every slice keeps >= 1536 of K (the runtime gives the slices 64 x 64 tiles; operands one
+//    element off: 1024 x 2048 x 8192 118 us in four slices, 131 whole, 2048 x 2048 x 4096 118 / 131).
 int64_t k_splits(const Plan& p) {
   if (p.batched || p.K % 64 != 0) return 1;
   int64_t s = 1;
@@ -133,6 +136,12 @@ int64_t k_splits(const Plan& p) {
   } else if (std::min(p.M, p.N) <= 64) {
     const int64_t tiles = ((p.M + 63) / 64) * ((p.N + 63) / 64), steps = p.K / 64;
     while (tiles * (2 * s) <= 256 && steps % (2 * s) == 0 && p.K / (2 * s) >= 128) s *= 2;
+  } else {
+    const int64_t wide = p.M % 128 == 0 && p.N % 256 == 0 ? (p.M / 128) * (p.N / 256) : 0;
+    const int64_t tall = p.M % 256 == 0 && p.N % 128 == 0 ? (p.M / 256) * (p.N / 128) : 0;
+    const int64_t blocks = std::max(wide, tall);
+    while (blocks * s < 192 && p.K % (64 * 2 * s) == 0 && p.K / (2 * s) >= 1536) s *= 2;
+    if (blocks * s < 192) s = 1;
   }
   return s;
 }
