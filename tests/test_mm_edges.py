@@ -249,6 +249,22 @@ def test_plan_query_agrees_with_the_workspace():
     assert plan_of(64, 64, 64, off=2).kernel == abi.MM_GENERAL
 
 
+# (m, n, k, ta, tb) that an earlier cost model put on a tile 12 to 24% slower than one it had (1152 x 1152 x 1024 on 64 x
+# 128 10.3 us, on 64 x 64 8.2), and the tiles within 10% of the fastest, all timed unsplit
+TILES = [((1152, 1152, 1024, False, False), {(64, 64)}), ((384, 2816, 2816, True, True), {(64, 64)}),
+         ((6144, 512, 1024, True, True), {(128, 128)}), ((5632, 512, 1920, True, True), {(128, 128)}),
+         ((8064, 384, 640, True, False), {(128, 128)}), ((1024, 2048, 2048, False, True), {(64, 128)}),
+         ((512, 3072, 3072, False, True), {(64, 128)}), ((1024, 1152, 1536, True, True), {(64, 64)}),
+         ((1472, 960, 320, False, False), {(64, 64)}), ((2176, 512, 2176, False, False), {(64, 64), (64, 128)}),
+         ((320, 4864, 1024, True, False), {(64, 64)}), ((1792, 832, 2944, True, False), {(64, 64), (64, 128)})]
+
+
+@pytest.mark.parametrize("product,tiles", TILES)
+def test_plan_takes_a_fast_tile(product, tiles):
+    p = plan_of(*product, split=False)
+    assert (p.tile_m, p.tile_n) in tiles
+
+
 def test_split_plan_on_the_host():
     """hrt_mm_workspace: whole numbers of [M, N] slices, none for full grids and products with kernels of their own,
     -1 for operands off 16-byte lines."""

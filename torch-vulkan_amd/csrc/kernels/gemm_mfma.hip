@@ -338,57 +338,53 @@ __global__ __launch_bounds__(256) void mm_dq8_mfma(hrt_mm_dq8_args p, int64_t ti
 }
 
 // ---- choice of tile and K split for the direct-to-LDS kernel -----------------------------------------------------
-// Cost model of mm_dma, in microseconds, fitted to event-timed products of 0.04 to 137 GFLOP whose operands come from
-// HBM (rotated through 600 MB; from a warm L2 the small tiles' steps take as little as two thirds).  A grid runs in
-// rounds of `slots` tiles (the workgroups that 256 CUs hold at once).  A K step of a round takes step[0] when the
-// chip is nearly empty; one workgroup per CU: rising to step[1] as the round fills (the tiles share L2 and power);
-// two or three per CU: step[l] with l + 1 workgroups on the fullest CU.  A round also takes its first loads (3 us
-// where nothing else runs on the CU meanwhile, else 1) and the writing of its outputs.  Measured / modelled:
-// 1024 x 8192 x 2048 NT on 128 x 256 tiles 38.6 / 38.6 us, 2048^3 on 128 x 128 24.5 / 24.5 (64 x 128 27.0 / 27.1),
-// 4096^3 on 256 x 256 122 / 122 (128 x 256 135), 1024 x 2048 x 2048 on 64 x 128 21.0 / 20.9 (64 x 64 22.2),
-// 1024 x 2048 x 6144 NN in four slices of 128 x 256 tiles 41.7 / 44 (64 x 128 unsplit 54.7), two products
-// 5760 x 8640 x 128 TT on 64 x 64 105 / 112 (256 x 256 116).
+// Cost model of mm_dma, in microseconds, fitted to 3225 products (all layouts, 2e-4 to 140 GFLOP, layers of 256 to 4096
+// tokens among them) timed on every tile and split, with operands from HBM (rotated through 600 MB) and from cache: what
+// it picks takes 1.8% longer than the best of them on average.  The numbers order the choices; as times they are rough.
+// A grid runs in rounds of `slots` tiles (the workgroups that 256 CUs hold at once).  A K step takes step[0] on a nearly
+// empty chip, step[i] when i workgroups a CU are at work and what lies between for part-filled rounds (the tiles share
+// L2 and power), kMasked times that in masked forms, whose last tiles hold less.  A round also takes its first loads and the
+// writing of its outputs.
 struct TileCost {
   uint32_t slots;
-  double step[3];
+  double first, step[4];
 };
 constexpr TileCost kTileCost[kGemmTiles] = {
-    {256, {1.19, 1.75}},         // 256 x 256
-    {256, {0.62, 1.00}},         // 128 x 256
-    {256, {0.62, 1.02}},         // 256 x 128
-    {256, {0.72, 0.79}},         // 128 x 192
-    {256, {0.50, 0.616}},        // 128 x 128
-    {512, {0.595, 0.76}},        // 64 x 128
-    {768, {0.47, 0.605, 0.62}},  // 64 x 64
+    {256, 3.12, {1.387, 2.029}},                 // 256 x 256
+    {256, 3.031, {0.6527, 1.156}},               // 128 x 256
+    {256, 1.854, {0.8738, 1.423}},               // 256 x 128
+    {256, 2.695, {0.6901, 0.8706}},              // 128 x 192
+    {256, 1.571, {0.4424, 0.7417}},              // 128 x 128
+    {512, 0.6518, {0.5139, 0.5901, 2.027}},      // 64 x 128
+    {768, 0.1275, {0.3852, 0.4836, 0.7293, 0.9727}}, // 64 x 64
 };
+constexpr double kMasked = 0.9717, kHalfLines = 1.178;
 
-double tile_us(const TileCost& c, TileShape sh, uint32_t tiles, uint32_t steps) {
+double tile_us(const TileCost& c, TileShape sh, uint32_t tiles, double steps) {
   const uint32_t full = tiles / c.slots, rest = tiles % c.slots;  // 32 bits: a plan costs a call well under 1 us
-  const double fill = (double)rest / c.slots, first = c.slots > 256 ? 1.0 : 3.0;
-  const double hi = c.step[c.slots > 256 ? c.slots / 256 - 1 : 1];
-  const double last = c.slots > 256 ? c.step[rest ? (rest - 1) / 256 : 0] : c.step[0] + (c.step[1] - c.step[0]) * fill;
-  const double out = 7.1 * (c.slots / 256) * sh.bm * sh.bn / 65536;  // a full round's outputs
-  double us = full * (first + out + steps * hi);
-  if (rest) us += first + out * fill + steps * last;
+  const double out = 5.499 * (c.slots / 256) * sh.bm * sh.bn / 65536;  // a full round's outputs
+  double us = full * (c.first + out + steps * c.step[c.slots / 256]);
+  if (rest) {
+    const uint32_t i = rest / 256;
+    const double last = c.step[i] + (c.step[i + 1] - c.step[i]) * (rest - 256 * i) / 256;
+    us += c.first + out * rest / c.slots + steps * last;
+  }
   return us;
 }
-// The partial products of a split: their write and read (at ~6 TB/s, a little of it lost to the tail of the slices),
-// the second launch, and each slice's start (1024 x 2048 x 8192, four slices: 10 us over the slices alone).  Charged at
-// 4.5 TB/s, 1024 x 2048 x 6144 NN went to two slices of 128 x 128 tiles, 42.6 us with their sum, instead of four of
-// 128 x 256, 41.1 (a DiT block's forward and backward 678.2 -> 675.9 us, a
-// 951 x 4928 x 1472 linear layer 92.9 -> 83.8; 7522 x 4352 x 256, whose weight gradient went from three slices to six,
-// 131.6 -> 134.7).
-double split_us(int64_t splits, int64_t M, int64_t N) { return 3.3 + 0.33 * splits + 0.85 * (double)splits * M * N * 4 / 5e6; }
+// The partial products of a split: their write and read, the second launch and each slice's start.
+double split_us(int64_t splits, int64_t M, int64_t N) { return 1.305 + 0.2128 * splits + 1.625 * (double)splits * M * N * 4 / 5e6; }
 
 struct GemmPlan {
   int tile = -1;  // GemmTile, -1: the direct-to-LDS kernel does not take the product
   int64_t splits = 1, kslice = 0;
+  double us = 0.0;
 };
 
 // The cheapest tile, and for one product (no batch) the cheapest number of K slices when may_split: under-filled
 // grids with a long reduction then run several slices per tile, whose fp32 partial products a second kernel adds
-// in order.  A split has to promise 8 us: its workspace and second launch cost the host 4 us, which a program of small
-// layers waits for.
+// in order.  A split has to promise kSplitGain: its workspace and second launch cost the host a few microseconds, which a
+// program of small layers waits for.
+constexpr double kSplitGain = 6.43;
 GemmPlan search_plan(const hrt_mm_args& a, bool may_split) {
   GemmPlan best, whole;
   const bool f32out = (a.flags & HRT_MM_F32_OUT) != 0;
@@ -402,35 +398,43 @@ GemmPlan search_plan(const hrt_mm_args& a, bool may_split) {
     if (t == T256x256 && (nk > 64 || nk < 8)) continue;  // its two-buffer ring waits a step for each copy: slower at 8192^3
     const int64_t tiles = cdiv(a.M, kTileShape[t].bm) * cdiv(a.N, kTileShape[t].bn) * a.batch;
     // a 64-wide tile of an operand contiguous along M or N whose rows start off 128-byte lines touches two lines for
-    // each line's worth (160 x 5000 x 5000 NN: 42 us on 64 x 64 tiles, 26 on 64 x 128)
+    // each line's worth
     const bool lines = (f.atr && kTileShape[t].bm == 64 && a.a_sk % 64 != 0) || (f.btr && kTileShape[t].bn == 64 && a.b_sk % 64 != 0);
+    const double slow = (lines ? kHalfLines : 1.0) * (f.exact ? 1.0 : kMasked);
     const bool slices_ok = t == T128x256 || t >= T128x128;  // tiles with an fp32-output form
     if (f32out && !slices_ok) continue;
     for (int s : kSplits) {
       // slices of at least 4 steps, and none that start a third round of tiles
       if (s > 1 && (!may_split || !slices_ok || a.batch != 1 || nk < 4 * s || tiles * s > 2 * kTileCost[t].slots)) break;
       const uint32_t per = (uint32_t)(nk + s - 1) / s, n = ((uint32_t)nk + per - 1) / per;
-      double us = (lines ? 1.25 : 1.0) * tile_us(kTileCost[t], kTileShape[t], tiles * n, per);
+      double us = tile_us(kTileCost[t], kTileShape[t], tiles * n, per * slow);
       if (n > 1) us += split_us(n, a.M, a.N);
-      const GemmPlan p{t, n, n > 1 ? (int64_t)per * GBK : 0};
+      const GemmPlan p{t, n, n > 1 ? (int64_t)per * GBK : 0, us};
       if (n == 1 && (whole.tile < 0 || us < whole_us)) whole_us = us, whole = p;
       if (best.tile < 0 || us < best_us) best_us = us, best = p;
     }
   }
-  return best.splits > 1 && whole.tile >= 0 && best_us > whole_us - 8.0 ? whole : best;
+  return best.splits > 1 && whole.tile >= 0 && best_us > whole_us - kSplitGain ? whole : best;
 }
 
-// The shim asks for a workspace and then queues the same product: the last plan is kept, by the values it depends on
-// (an unsplit choice among splits is the choice without them too).
+// The shim asks for a workspace and then queues the same product, and a program's layers come back: the plans of the
+// last few dozen products are kept per thread, by the values they depend on (an unsplit choice among splits is the choice
+// without them too).  A search takes 0.35 to 0.55 us of the host's 4 per product, a kept plan 0.05.
 GemmPlan plan_gemm(const hrt_mm_args& a, bool may_split) {
+  struct Kept {
+    std::array<int64_t, 17> key{};  // M = 0: no plan yet
+    GemmPlan plan;
+    bool split = false;
+  };
   const std::array<int64_t, 17> key = {a.M, a.N, a.K, a.batch, a.a_sb, a.a_sm, a.a_sk, a.b_sb, a.b_sk, a.b_sn, a.c_sb, a.c_sm, a.c_sn,
                                        (int64_t)(a.a % 16), (int64_t)(a.b % 16), (int64_t)(a.c % 16), (int64_t)a.flags};
-  thread_local std::array<int64_t, 17> last_key{};  // M = 0: no plan yet
-  thread_local GemmPlan last;
-  thread_local bool last_split = false;
-  if (key != last_key || (may_split != last_split && !(last_split && last.splits == 1)))
-    last = search_plan(a, may_split), last_key = key, last_split = may_split;
-  return last;
+  uint64_t h = 0;
+  for (const int64_t x : key) h = (h ^ (uint64_t)x) * 0x9e3779b97f4a7c15ull;
+  thread_local std::array<Kept, 64> kept;
+  Kept& e = kept[h >> 58];
+  if (key != e.key || (may_split != e.split && !(e.split && e.plan.splits == 1)))
+    e.plan = search_plan(a, may_split), e.key = key, e.split = may_split;
+  return e.plan;
 }
 
 // Which loader an operand can use.  rows = M (A) or N (B); s_r / s_k its strides.
@@ -521,14 +525,14 @@ void queue_dq8(const hrt_mm_dq8_args& a, hipStream_t s) {
   hipLaunchKernelGGL((mm_dq8_mfma<T, BM, BN, 2, 2, AM>), dim3((uint32_t)(tm * tn)), dim3(256), 0, s, a, tm, tn);
 }
 
-// The same choice for the fused int8 linear (tile costs include the conversion of the int8 tile: M = 512 at 8192 x 2048
+// The same choice for the fused int8 linear (tile costs, fitted to 237 products, include the conversion of the int8 tile: M = 512 at 8192 x 2048
 // weights 31 us on 128 x 128 tiles, 41 on 256 x 128, 50 on 64 x 64; M = 16 on 64 x 64 12 us in four slices, 19 unsplit).  A split keeps its partial products in the optional workspace, which a caller may size for the
 // dequantized weights: N K 16-bit elements hold them while 2 splits M <= K.
 GemmPlan plan_dq8(const hrt_mm_dq8_args& d, bool may_split) {
   static constexpr struct {
     GemmTile t;
     TileCost c;
-  } kTiles[] = {{T256x128, {256, {0.80, 1.30}}}, {T128x128, {256, {0.60, 0.83}}}, {T64x64, {768, {0.52, 0.68, 0.90}}}};
+  } kTiles[] = {{T256x128, {256, 2.256, {0.7299, 1.526}}}, {T128x128, {256, 0.8656, {0.8287, 1.019}}}, {T64x64, {768, 0.01143, {0.6201, 0.6693, 0.914, 1.166}}}};
   GemmPlan best;
   if (d.K % GBK || d.q % 16 || d.scale % 2) return best;
   const hrt_mm_args a = dq8_as_mm(d);
@@ -542,8 +546,8 @@ GemmPlan plan_dq8(const hrt_mm_dq8_args& d, bool may_split) {
       if (s > 1 && (!may_split || k.t != T64x64 || nk < 4 * s || 2 * s * d.M > d.K)) break;
       const int64_t per = cdiv(nk, s), n = cdiv(nk, per);
       double us = tile_us(k.c, kTileShape[k.t], tiles * n, per);
-      if (n > 1) us = 1.05 * (us + split_us(n, a.M, a.N));
-      if (best.tile < 0 || us < best_us) best_us = us, best = GemmPlan{k.t, n, n > 1 ? per * GBK : 0};
+      if (n > 1) us += 3.697 + split_us(n, a.M, a.N);
+      if (best.tile < 0 || us < best_us) best_us = us, best = GemmPlan{k.t, n, n > 1 ? per * GBK : 0, us};
     }
   }
   return best;
@@ -566,6 +570,11 @@ hrt_mm_args dq8_weights_as_mm(const hrt_mm_dq8_args& d) {
 // converts every weight once per 256-row block of x, which costs more than one standalone dequant pass
 // beyond a few blocks (M = 4096: 222 us fused vs ~157 us dequant + GEMM for 8192 x 2048 weights).
 constexpr int64_t kDq8WsMinM = 2048;
+// The plan of the product on dequantized weights (ws: their address, 0 = any aligned one), tile = -1: the fused kernel.
+GemmPlan plan_dequant(const hrt_mm_dq8_args& d) {
+  if (d.M < kDq8WsMinM || d.K % GBK != 0) return GemmPlan{};
+  return plan_gemm(dq8_weights_as_mm(d), false);
+}
 
 template <typename T>
 bool launch_mm_dq8(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
@@ -579,23 +588,20 @@ bool launch_mm_dq8(const void* pp, const uint32_t*, hrt::LaunchCtx& ctx) {
       !ctx.check(a.scale, (uint64_t)(a.N * a.nblocks) * 2, "scale") || !ctx.check(a.y, (uint64_t)(a.M * a.N) * 2, "y") ||
       (a.has_bias && !ctx.check(a.bias, (uint64_t)a.N * 2, "bias")))
     return false;
-  // large M with a workspace: dequantize once (the dq8 kernel), then the fast GEMM on the bf16 / f16 weights
+  // many rows and a workspace: dequantize once (the dq8 kernel), then the GEMM on the bf16 / f16 weights, where faster
   const bool ws_ok = a.ws && a.ws % 16 == 0;
-  if (ws_ok && a.M >= kDq8WsMinM && a.K % GBK == 0) {
+  if (const GemmPlan plan = ws_ok ? plan_dequant(a) : GemmPlan{}; plan.tile >= 0) {
     const hrt_mm_args m = dq8_weights_as_mm(a);
-    const GemmPlan plan = plan_gemm(m, false);
-    if (plan.tile >= 0) {
-      if (!ctx.check(a.ws, (uint64_t)(a.N * a.K) * 2, "ws")) return false;
-      hrt_dq8_args d{};
-      d.q = a.q, d.scale = a.scale, d.out = a.ws, d.rows = a.N, d.cols = a.K, d.nblocks = a.nblocks;
-      const char* dq = std::is_same<T, BF16>::value ? "dq8_bf16" : "dq8_f16";
-      for (auto& e : hrt::kernel_table())
-        if (!strcmp(e.name, dq)) {
-          if (!e.launch(&d, nullptr, ctx)) return false;
-          if (dma_queue<T>(m, (GemmTile)plan.tile, 0, ctx.stream)) return hrt::launch_ok(hipGetLastError(), ctx, "mm_dq8_ws");
-        }
-      return ctx.fail("mm_dq8: workspace path unavailable");
-    }
+    if (!ctx.check(a.ws, (uint64_t)(a.N * a.K) * 2, "ws")) return false;
+    hrt_dq8_args d{};
+    d.q = a.q, d.scale = a.scale, d.out = a.ws, d.rows = a.N, d.cols = a.K, d.nblocks = a.nblocks;
+    const char* dq = std::is_same<T, BF16>::value ? "dq8_bf16" : "dq8_f16";
+    for (auto& e : hrt::kernel_table())
+      if (!strcmp(e.name, dq)) {
+        if (!e.launch(&d, nullptr, ctx)) return false;
+        if (dma_queue<T>(m, (GemmTile)plan.tile, 0, ctx.stream)) return hrt::launch_ok(hipGetLastError(), ctx, "mm_dq8_ws");
+      }
+    return ctx.fail("mm_dq8: workspace path unavailable");
   }
   // K in whole steps: dequant fused into the direct-to-LDS GEMM, K split over the workspace where the grid is small
   const GemmPlan plan = plan_dq8(a, ws_ok);
@@ -777,7 +783,7 @@ extern "C" int64_t hrt_mm_workspace(const hrt_mm_args* a, int32_t dtype) {
 
 extern "C" int64_t hrt_mm_dq8_workspace(const hrt_mm_dq8_args* a) {
   if (a == nullptr || a->M <= 0 || a->N <= 0 || a->K <= 0) return 0;
-  if (a->M >= hk::kDq8WsMinM) return a->N * a->K;
+  if (hk::plan_dequant(*a).tile >= 0) return a->N * a->K;
   // not N K: 256 MiB and more is a reservation and a wait for the GPU on every call (16 x 16384 x 8192 340 us, 41 so)
   const int64_t splits = hk::plan_dq8(*a, true).splits;
   return splits > 1 ? 2 * splits * a->M * a->N : 0;  // fp32 partial products in 16-bit elements
@@ -803,13 +809,10 @@ extern "C" int hrt_mm_plan_of(const hrt_mm_args* a, int32_t dtype, int32_t may_s
 extern "C" int hrt_mm_dq8_plan_of(const hrt_mm_dq8_args* a, int32_t with_ws, hrt_mm_plan* out) {
   if (a == nullptr || out == nullptr || a->M <= 0 || a->N <= 0 || a->K <= 0) return -1;
   *out = hrt_mm_plan{HRT_MM_GENERAL, 64, 64, 0, 1};
-  if (with_ws != 0 && a->M >= hk::kDq8WsMinM && a->K % hk::GBK == 0) {
-    const hrt_mm_args m = hk::dq8_weights_as_mm(*a);
-    hk::fill_plan(m, hk::plan_gemm(m, false), out);
-    if (out->kernel == HRT_MM_DIRECT) {
-      out->kernel = HRT_MM_DEQUANT;
-      return 0;
-    }
+  if (const hk::GemmPlan p = with_ws != 0 ? hk::plan_dequant(*a) : hk::GemmPlan{}; p.tile >= 0) {
+    hk::fill_plan(hk::dq8_weights_as_mm(*a), p, out);
+    out->kernel = HRT_MM_DEQUANT;
+    return 0;
   }
   hk::fill_plan(hk::dq8_as_mm(*a), hk::plan_dq8(*a, with_ws != 0), out);
   return 0;
