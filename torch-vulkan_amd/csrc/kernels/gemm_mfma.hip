@@ -570,10 +570,13 @@ hrt_mm_args dq8_weights_as_mm(const hrt_mm_dq8_args& d) {
 // converts every weight once per 256-row block of x, which costs more than one standalone dequant pass
 // beyond a few blocks (M = 4096: 222 us fused vs ~157 us dequant + GEMM for 8192 x 2048 weights).
 constexpr int64_t kDq8WsMinM = 2048;
-// The plan of the product on dequantized weights (ws: their address, 0 = any aligned one), tile = -1: the fused kernel.
+// The plan of the product on dequantized weights (ws: their address, 0 = any aligned one) where that is estimated
+// faster, with the pass that dequantizes them, than the fused kernel; else tile = -1.  Short reductions stay fused: 2048 x
+// 1024 x 320 7.1 us against 8.8, 3120 x 1024 x 320 8.1 / 10.0, 2048 x 2048 x 2048 33.1 / 30.4.
 GemmPlan plan_dequant(const hrt_mm_dq8_args& d) {
   if (d.M < kDq8WsMinM || d.K % GBK != 0) return GemmPlan{};
-  return plan_gemm(dq8_weights_as_mm(d), false);
+  const GemmPlan whole = plan_gemm(dq8_weights_as_mm(d), false), fused = plan_dq8(d, false);
+  return whole.tile >= 0 && (fused.tile < 0 || whole.us + 2.0 < fused.us) ? whole : GemmPlan{};
 }
 
 template <typename T>
