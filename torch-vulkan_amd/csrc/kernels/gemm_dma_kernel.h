@@ -57,7 +57,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void mm_dma(hrt_mm_args
                                                                    uint64_t dq_scale, int64_t dq_nblocks,
                                                                    int64_t kslice) {
   static_assert(!DQ8 || !BTR, "int8 B is staged as [n][k] rows");
-  static_assert(RING == 3 || (RING >= 2 && RING <= 6 && !DQ8), "three-buffer ring, or 2 to 6 buffers for the plain GEMM");
+  static_assert(RING == 3 || (RING == 2 && !DQ8), "three-buffer ring, or two buffers for the plain GEMM");
   constexpr int WNN = BN / WN;         // wavefronts along n
   constexpr int NW = (BM / WM) * WNN;  // wavefronts
   constexpr int FM = WM / 32, FN = WN / 32;  // 32 x 32 accumulators per wavefront along m, n
@@ -81,20 +81,17 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void mm_dma(hrt_mm_args
   __shared__ __attribute__((aligned(1024))) uint8_t a0_raw[A_TILE], a1_raw[A_TILE], a2_raw[RING >= 3 ? A_TILE : 16];
   __shared__ __attribute__((aligned(1024))) uint8_t b0_raw[B_TILE], b1_raw[B_TILE];
   __shared__ __attribute__((aligned(1024))) uint8_t b2_raw[DQ8 ? Q_TILE : RING >= 3 ? B_TILE : 16];  // DQ8: int8 tile 0
-  __shared__ __attribute__((aligned(1024))) uint8_t a3_raw[RING >= 4 ? A_TILE : 16], b3_raw[RING >= 4 ? B_TILE : 16];
-  __shared__ __attribute__((aligned(1024))) uint8_t a4_raw[RING >= 5 ? A_TILE : 16], b4_raw[RING >= 5 ? B_TILE : 16];
-  __shared__ __attribute__((aligned(1024))) uint8_t a5_raw[RING >= 6 ? A_TILE : 16], b5_raw[RING >= 6 ? B_TILE : 16];
   __shared__ __attribute__((aligned(DQ8 ? 1024 : 16))) uint8_t q1_raw[Q_TILE], q2_raw[Q_TILE];
   HK_L uint8_t* const A0 = (HK_L uint8_t*)a0_raw;
   HK_L uint8_t* const A1 = (HK_L uint8_t*)a1_raw;
   HK_L uint8_t* const B0 = (HK_L uint8_t*)b0_raw;
   auto abuf = [&](auto ic) {
     constexpr int I = decltype(ic)::value;
-    return (HK_L uint8_t*)(I == 0 ? a0_raw : I == 1 ? a1_raw : I == 2 ? a2_raw : I == 3 ? a3_raw : I == 4 ? a4_raw : a5_raw);
+    return (HK_L uint8_t*)(I == 0 ? a0_raw : I == 1 ? a1_raw : a2_raw);
   };
   auto bbuf = [&](auto ic) {
     constexpr int I = decltype(ic)::value;
-    return (HK_L uint8_t*)(I == 0 ? b0_raw : I == 1 ? b1_raw : I == 2 ? b2_raw : I == 3 ? b3_raw : I == 4 ? b4_raw : b5_raw);
+    return (HK_L uint8_t*)(I == 0 ? b0_raw : I == 1 ? b1_raw : b2_raw);
   };
   HK_L uint8_t* const Q0 = (HK_L uint8_t*)b2_raw;
   HK_L uint8_t* const Q1 = (HK_L uint8_t*)q1_raw;
@@ -620,7 +617,6 @@ bool dma_queue_dq8(const hrt_mm_dq8_args& d, GemmTile tile, uint64_t ws, int64_t
   return true
   switch (tile) {
     case T256x128: HK_TILE(256, 128, 64, 64);
-    case T128x256: HK_TILE(128, 256, 64, 64);
     case T128x128: HK_TILE(128, 128, 32, 64);
     case T64x64: HK_TILE(64, 64, 32, 32);
     default: return false;
