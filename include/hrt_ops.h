@@ -402,18 +402,20 @@ static inline int64_t hrt_conv3_splits(int64_t N, int64_t I, int64_t O, int64_t 
  * output rows x 32 pixels per workgroup, the last block of output channels padded to 128 by zero rows of wr, which
  * holds hrt_conv3r_wr_bytes(O, I) bytes. */
 static inline int64_t hrt_conv3r_wr_bytes(int64_t O, int64_t I) { return hrt_conv3_wr_bytes((O + 127) / 128 * 128, I); }
-/* Input-channel split of "conv3x3r_{dt}": the cheapest of the divisors of I / 16 that leave 4 channel blocks, a round
- * of 256 workgroups taking ~1.6 us a block and a split its partial sums' write and read and a launch. */
+/* Estimated time of "conv3x3r_*" over `splits` slices of the input channels, in us: rounds of 256 workgroups at ~1.6 a
+ * channel block and 3.5 for a round's first loads and its outputs, 5 for the launch and the weights' reordering, and
+ * for slices the write and read of their partial sums and a launch. */
+static inline double hrt_conv3r_us(int64_t N, int64_t I, int64_t O, int64_t H, int64_t W, int64_t splits) {
+  const int64_t tiles = N * ((H + 3) / 4) * ((W + 31) / 32) * ((O + 127) / 128), blocks = I / 16 / splits;
+  const double us = (double)((tiles * splits + 255) / 256) * (1.6 * (double)blocks + 3.5) + 5.0;
+  return splits > 1 ? us + 3.0 + 1.3e-6 * (double)(splits * N * O) * (double)(H * W) : us;
+}
+/* Input-channel split of "conv3x3r_{dt}": the cheapest of the divisors of I / 16 that leave 4 channel blocks. */
 static inline int64_t hrt_conv3r_splits(int64_t N, int64_t I, int64_t O, int64_t H, int64_t W) {
-  const int64_t tiles = N * ((H + 3) / 4) * ((W + 31) / 32) * ((O + 127) / 128), nb = I / 16;
+  const int64_t nb = I / 16;
   int64_t best = 1;
-  double best_us = 0.0;
-  for (int64_t s = 1; s <= 8 && (s == 1 || nb / s >= 4); ++s) {
-    if (nb % s != 0) continue;
-    double us = (double)((tiles * s + 255) / 256) * (double)(nb / s) * 1.6;
-    if (s > 1) us += 3.0 + 1.3e-6 * (double)(s * N * O) * (double)(H * W);
-    if (s == 1 || us < best_us) best_us = us, best = s;
-  }
+  for (int64_t s = 2; s <= 8 && nb / s >= 4; ++s)
+    if (nb % s == 0 && hrt_conv3r_us(N, I, O, H, W, s) < hrt_conv3r_us(N, I, O, H, W, best)) best = s;
   return best;
 }
 typedef struct hrt_conv3_wprep_args {

@@ -90,9 +90,8 @@ at::Tensor cols_of(const at::Tensor& input, const ConvShape& g) {
 // aligned addresses only (a view at an odd offset, e.g. a weight inside a flat parameter buffer, goes to the
 // unfolding + GEMM path, which takes any alignment).
 // Which form of the direct kernel: kExact above; kRagged ("conv3x3r_{dt}") for output channels in multiples of 32 from
-// 128 and rows of a multiple of 8 pixels, where an estimate of its time (rounds of 256 workgroups, ~1.6 us a channel
-// block, padding included) is 5% below that of the unfolding (the column matrix at 2.8 TB/s, its adjoint at 2.2, the
-// product at 600 TFLOP/s).  Measured, direct against unfolded, forward / input gradient: 512 -> 320 on 96 x 96 58 / 62
+// 128 and rows of a multiple of 8 pixels, where an estimate of its time (hrt_conv3r_us, padding included) is 5% below
+// that of the unfolding (the column matrix at 2.8 TB/s, its adjoint at 2.2, the product at 600 TFLOP/s).  Measured, direct against unfolded, forward / input gradient: 512 -> 320 on 96 x 96 58 / 62
 // against 82 / 77 us, two 640 -> 128 on 120 x 72 71 / 66 against 109 / 138, 320 -> 320 on 64 x 64 30 / 29 against 46 / 27;
 // two 128 -> 640 on 120 x 72 stay unfolded forward (73 against 65).
 enum class Direct { kNo, kExact, kRagged };
@@ -105,10 +104,8 @@ Direct conv3_form(const ConvShape& g, at::ScalarType t, int64_t in_ch, int64_t o
     return Direct::kNo;
   if (out_ch % 128 == 0 && g.W % 64 == 0) return Direct::kExact;
   if (out_ch % 32 != 0 || out_ch < 128 || g.W % 8 != 0) return Direct::kNo;
-  const int64_t S = hrt_conv3r_splits(g.N, in_ch, out_ch, g.H, g.W);
-  const int64_t tiles = g.N * ((g.H + 3) / 4) * ((g.W + 31) / 32) * ((out_ch + 127) / 128) * S;
-  const double px = (double)(g.N * g.H) * g.W, split = S > 1 ? 3.0 + 1.3e-6 * S * out_ch * px : 0.0;
-  const double direct = (double)((tiles + 255) / 256) * (1.6 * in_ch / 16 / S + 3.5) + 5.0 + split;
+  const double direct = hrt_conv3r_us(g.N, in_ch, out_ch, g.H, g.W, hrt_conv3r_splits(g.N, in_ch, out_ch, g.H, g.W));
+  const double px = (double)(g.N * g.H) * g.W;
   const double product = 18.0 * in_ch * out_ch * px / 600e6 + 6.0, columns = 18e-6 * g.C * px;  // us; MB
   const double unfolded = product + (adjoint ? 4.0 + columns / 2.2 : 8.0 + columns / 2.8);
   return 1.05 * direct < unfolded ? Direct::kRagged : Direct::kNo;
