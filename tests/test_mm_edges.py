@@ -216,6 +216,28 @@ def test_infinities_and_nans_stay_in_their_rows():
     assert torch.equal(torch.isnan(out), torch.isnan(ref)) and torch.equal(torch.isinf(out), torch.isinf(ref))
 
 
+@gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(130, 136, 72), (256, 256, 128), (70, 72, 1096)])
+def test_expanded_operands(m, n, k, dt):
+    """Operands repeated along M, N or K by a zero stride, against the same values laid out."""
+    g = torch.Generator().manual_seed(m + k)
+
+    def forms(rows, cols):
+        full, row, col = (torch.randn(s, generator=g).to(dt).to(dev) for s in ((rows, cols), (1, cols), (rows, 1)))
+        return full, row.expand(rows, cols), col.expand(rows, cols), row[:, :1].expand(rows, cols)
+
+    for i, A in enumerate(forms(m, k)):
+        for j, B in enumerate(forms(k, n)):
+            if i == j == 0:
+                continue
+            a, b = A.cpu().double(), B.cpu().double()
+            out = torch.mm(A, B).cpu().double()
+            # roundings of repeated values do not average out: k of them, each of the sum of the sizes of the terms
+            bound = (a.abs() @ b.abs()) * (2.0**-23 * k) + (out.abs() * (2.0**-8 if dt == torch.bfloat16 else 2.0**-23))
+            assert ((out - a @ b).abs() <= bound + 1e-30).all(), (i, j)
+
+
 def plan(m, n, k, a_off=0, dtype=abi.BF16, **kw):
     lib = ctypes.CDLL(abi._LIB_PATH)
     lib.hrt_mm_workspace.restype = ctypes.c_int64
