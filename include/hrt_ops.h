@@ -205,11 +205,12 @@ int hrt_mm_plan_of(const hrt_mm_args* mm, int32_t dtype, int32_t may_split, hrt_
  *   deq(q)[n, k] = round_dtype(float(q[n, k]) * float(scale[n, k / 64]))      (bit-exact dequant value)
  * x: [M, K] with strides (x_sm, x_sk); q: int8 [N, K] contiguous; scale: bf16 [N, nblocks] contiguous,
  * nblocks = ceil(K / 64); bias: [N] (if has_bias); y: [M, N] contiguous, dtype of x.
- * ws (optional, 0 = none): 16-byte aligned workspace of N * K elements of x's dtype.  For large M (the
- * weights would otherwise be converted once per 256-row block of x) the weights are dequantized into it
- * once and the product runs on them; the values are the same either way.  For small M it may hold fp32 partial
- * products over slices of K, added in order (a reduction order of its own).  hrt_mm_dq8_workspace gives the
- * elements that help a call: N * K, the size of those partial products (at most N * K), or 0. */
+ * ws (optional, 0 = none): 16-byte aligned workspace of N * K elements of x's dtype, or of the elements that
+ * hrt_mm_dq8_workspace gives.  For many rows (the weights would otherwise be converted once per 256-row block of x) the
+ * weights are dequantized into it once, where that is estimated faster, and the product runs on them; for few it holds
+ * fp32 partial products over slices of K, added in order.  The weights' values are the same either way; the order of
+ * the fp32 sums over K is each form's own.  hrt_mm_dq8_workspace: N * K, the size of the partial products (at most
+ * N * K), or 0 where a workspace does not help. */
 typedef struct hrt_mm_dq8_args {
   uint64_t x, q, scale, bias, y;
   int64_t M, N, K, nblocks;

@@ -733,7 +733,8 @@ constexpr int QST = 128;  // queries per LDS stage of the dK / dV kernel
 // PAD: as the forward's.  SPLIT: few key blocks (a 77-token context: two per head) would leave most CUs idle, so
 // `splits` workgroups share a key block, each taking a run of query stages and writing fp32 partial dK, dV
 // ([split][b h][key][2][D] in p.o32) that attn_dkdv_sum adds in split order (B2 H8, 1024 queries, 77 keys of 80: 56 us
-// on 32 workgroups of the general kernel; the whole forward + backward 88 -> 43).
+// on 32 workgroups of the general kernel, 19.1 on as many here, 14.3 with the sum in eight ranges; forward + backward
+// through autograd 88 -> 40 to 47 us, of which the kernels take 31 and the host the rest).
 template <typename T, int DCH, bool PAD, bool SPLIT>
 __global__ __launch_bounds__(512) void attn_dkdv_w32(hrt_attn_args p, int nkb, int splits) {
   constexpr int NW = 8;
@@ -1120,10 +1121,12 @@ __global__ __launch_bounds__(256) void attn_dkdv_sum(hrt_attn_args p, int splits
 }
 
 // Query splits of the fast dK / dV path: as many as keep its workgroups within one round of 256, whole 128-query stages
-// each.  A split costs its partials' write and read and a launch (5 - 7 us); a stage that a workgroup no longer walks
-// saves ~1.1 us in 128-wide tiles and ~0.8 in 64-wide ones.  Forward + backward unsplit / split: 588 keys of 128, B3 H1,
-// 896 queries (6 stages saved) 39.6 / 42.0 us, 1408 (10) 45.4 / 42.2, 2048 (15) 54.5 / 45.3; 77 keys of 80, B2 H8,
-// 1024 queries (7) 35.3 / 33.6; keys of 64, H8: 300 and 1024 queries (7) 31.7 / 33.2, 500 and 2048 (12) 40.4 / 36.1.
+// each.  A split costs its partials' write and read and a launch (4 - 9 us by their size); a stage that a workgroup no
+// longer walks saves 1.4 us in 128-wide tiles and 1.0 in 64-wide ones.  Kernels queued back to back, 252 shapes of 16 to
+// 80 key blocks, 384 to 4096 queries: from 7 saved stages of 128-wide tiles a split changes the time by +1.2 us (B1 H8, 500
+// keys of 128: 20.9 / 22.2) to -6.0 (B1 H8, 77 keys of 80: 19.1 / 13.0), from 10 of 64-wide ones by -4.2 (B1 H8, 300 keys of
+// 64: 18.5 / 14.3) and more, from 4 saved stages by 0 to -2 where the blocks are few.  The lines lie above that crossing
+// since a split also costs the host a workspace and a launch (~4 us), which small layers wait for.
 int dkdv_splits(const hrt_attn_args& a) {
   const int64_t wgs = (int64_t)((a.Sk + 63) / 64) * a.B * a.H, nst = (a.Sq + QST - 1) / QST;
   if (wgs > 128) return 1;

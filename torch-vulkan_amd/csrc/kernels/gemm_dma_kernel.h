@@ -19,9 +19,12 @@
 // EDGE: sizes that are no multiple of the tile or of a K step.  The copies go through a buffer resource whose range
 // check returns zeros for the lanes past an edge (edge_lane_offsets), the partial K step comes first, so that the
 // loop itself masks nothing, and the epilogue stores what exists.  The products of M = 4020 tokens (2048 x 2048
-// weights) took 66 / 89 / 133 us (x W^T, g W, g^T x) in the register-staged general kernel (gemm_mfma.hip) and take
-// 37 / 37 / 45; on whole tiles the form is within 4% of the exact one either way, which stays for the 128 x 256
-// tiles' 3%.
+// weights, cold) took 66 / 89 / 133 us (x W^T, g W, g^T x) in the register-staged general kernel (gemm_mfma.hip) and take
+// 37.4 / 38.4 / 44.3 (34.6 / 35.5 / 38.8 from cache).  The exact form stays for whole tiles: 4096 x 4096 x 2048 against
+// 4088 x 4088 x 2048 takes 66.3 / 68.1 us (NT), 66.0 / 70.8 (NN), 65.5 / 71.2 (TN), 66.4 / 70.3 (TT); with half the M
+// or N the two are within 5% either way.  Tile indices are read back into scalar registers (readfirstlane): from the
+// vector registers that their divisions leave them in, every copy was a loop over distinct resources (806 x 4096 x 3840
+// 45.8 us so, 41.3 now).
 //
 // DQ8 (the fused int8 linear y = x deq(q)^T + bias): B is int8 q [N][K] with one bf16 scale per row and
 // 64-column block, so a K step covers exactly one scale block.  The raw int8 rows of step kt + 3 are copied

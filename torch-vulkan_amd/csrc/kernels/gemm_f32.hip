@@ -15,7 +15,7 @@
 //   * edges: lanes past M, N or K read zeros by the buffer's range check, the partial K step comes first (as
 //     gemm_dma_kernel.h).
 // Measured: 4096^3 NT 975 us, 141 TFLOP/s; x W^T / g W / g^T x of 1024 tokens, 1024 -> 2048: 141 / 187 / 325 us in the
-// scalar kernel (gemm.hip), 45 / 51 / 46 here; relative L2 error against float64 the same (5.7e-7 at K = 1024).
+// scalar kernel (gemm.hip), 39.0 / 46.7 / 40.2 here (the layer 659 -> 136.6); relative L2 error against float64 the same (5.7e-7 at K = 1024).
 #include <type_traits>
 #include <utility>
 
@@ -215,7 +215,7 @@ void queue_f32(const hrt_mm_args& a, bool atr, bool btr, int64_t kslice, hipStre
 }
 
 constexpr int FT = 64;  // tile edge: 128 x 128 tiles (eight wavefronts of 64 x 32) were slower everywhere (1024 x 2048 x
-                        // 1024 73 against 45 us, half the CUs idle; 4096^3 1026 against 975)
+                        // 1024 73 against 45 us traced, half the CUs idle; 4096^3 1026 against 975)
 
 // Whether a tile's element offsets fit the copies' 31 bits.
 bool f32_fits(const hrt_mm_args& a) {
@@ -272,7 +272,7 @@ int64_t f32_splits(const hrt_mm_args& a) {
     if (s == 1) whole_us = us;
     if (s == 1 || us < best_us) best_us = us, best = n;
   }
-  return best_us > whole_us - 8.0 ? 1 : best;  // 8 us: as the 16-bit plan (gemm_mfma.hip)
+  return best_us > whole_us - 8.0 ? 1 : best;  // the workspace and the second launch cost the host ~4 us, the estimate is rough
 }
 
 // c = alpha * (sum of the slices in order) + beta * bias, four outputs per thread.

@@ -525,8 +525,9 @@ void queue_dq8(const hrt_mm_dq8_args& a, hipStream_t s) {
   hipLaunchKernelGGL((mm_dq8_mfma<T, BM, BN, 2, 2, AM>), dim3((uint32_t)(tm * tn)), dim3(256), 0, s, a, tm, tn);
 }
 
-// The same choice for the fused int8 linear (tile costs, fitted to 237 products, include the conversion of the int8 tile: M = 512 at 8192 x 2048
-// weights 31 us on 128 x 128 tiles, 41 on 256 x 128, 50 on 64 x 64; M = 16 on 64 x 64 12 us in four slices, 19 unsplit).  A split keeps its partial products in the optional workspace, which a caller may size for the
+// The same choice for the fused int8 linear (tile costs, fitted to 237 products, include the conversion of the int8 tile:
+// M = 512 at 8192 x 2048 weights 31 us on 128 x 128 tiles, 41 on 256 x 128, 50 on 64 x 64; M = 16 on 64 x 64 12 us in four
+// slices, 19 unsplit).  A split keeps its partial products in the optional workspace, which a caller may size for the
 // dequantized weights: N K 16-bit elements hold them while 2 splits M <= K.
 GemmPlan plan_dq8(const hrt_mm_dq8_args& d, bool may_split) {
   static constexpr struct {
@@ -566,9 +567,9 @@ hrt_mm_args dq8_weights_as_mm(const hrt_mm_dq8_args& d) {
   return m;
 }
 
-// Smallest M at which the fused int8 linear dequantizes into the caller's workspace first: the fused kernel
+// Smallest M at which the fused int8 linear may dequantize into the caller's workspace first: the fused kernel
 // converts every weight once per 256-row block of x, which costs more than one standalone dequant pass
-// beyond a few blocks (M = 4096: 222 us fused vs ~157 us dequant + GEMM for 8192 x 2048 weights).
+// beyond a few blocks (M = 4096: 222 us fused vs 153 us dequant + GEMM for 8192 x 2048 weights).
 constexpr int64_t kDq8WsMinM = 2048;
 // The plan of the product on dequantized weights (ws: their address, 0 = any aligned one) where that is estimated
 // faster, with the pass that dequantizes them, than the fused kernel; else tile = -1.  Short reductions stay fused: 2048 x
